@@ -7,12 +7,13 @@ sources, so the built file travels with the source tree.
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "libstile_hip.so")
-SOURCES = ["stile_kernels.hip", "stile_plan.hip"]
+SOURCES = ["stile_kernels.hip", "stile_attention.hip", "stile_plan.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
@@ -29,12 +30,10 @@ COMMON_FLAGS = [
 def build_native(verbose=False):
     """Compile every HIP source and link libstile_hip.so (always rebuilds)."""
     os.makedirs(LIB_DIR, exist_ok=True)
-    objs = []
-    for src in SOURCES:
-        obj = os.path.join(LIB_DIR, os.path.splitext(src)[0] + ".o")
-        cmd = [HIPCC, *COMMON_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
-        _run(cmd, verbose)
-        objs.append(obj)
+    objs = [os.path.join(LIB_DIR, os.path.splitext(src)[0] + ".o") for src in SOURCES]
+    cmds = [[HIPCC, *COMMON_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj] for src, obj in zip(SOURCES, objs)]
+    with ThreadPoolExecutor(4) as pool:   # the sources compile side by side
+        list(pool.map(lambda cmd: _run(cmd, verbose), cmds))
     tmp = LIB_PATH + ".tmp"
     _run([HIPCC, "-shared", f"--offload-arch={ARCH}", "-fPIC", *objs, "-o", tmp], verbose)
     os.replace(tmp, LIB_PATH)

@@ -150,6 +150,15 @@ struct SpmmPlanDev {
   const int32_t* lds_xcd_host;
 };
 
+// Launch order of the fused attention kernel: win[] lists the plan's windows
+// by first row (so by matrix), and XCD x takes [start[x], start[x + 1]) of it
+// (cut at equal estimated cost), so that the K and V rows of the few masks an
+// XCD works on at a time stay in its 4 MB L2.
+struct AttOrder {
+  const int32_t* win;
+  int32_t start[kXcds + 1];
+};
+
 // Device view of a hybrid SDDMM plan.
 //   1D part: n1d entries (row, col, out) computed as FP32 dot products.
 //   Block part: nblk 16x16 output blocks: rows blk_rows[b][16],
@@ -201,8 +210,8 @@ hipError_t launch_set_values(const SpmmPlanDev& p, const float* vals, const int3
                              const int32_t* res_ids, int64_t n_res, const int32_t* sp_ids, int64_t n_sp,
                              hipStream_t s);
 
-hipError_t launch_attention(const SpmmPlanDev& p, const void* Q, const void* K, const void* V, int64_t ld,
-                            float scale, float* out, int64_t ldo, hipStream_t s);
+hipError_t launch_attention(const SpmmPlanDev& p, const AttOrder& ord, const void* Q, const void* K, const void* V,
+                            int64_t ld, float scale, float* out, int64_t ldo, hipStream_t s);
 hipError_t launch_ell_bucket_spmm(int rows, int width, const int32_t* orow, const int32_t* cols, const float* vals,
                                   const float* B, int64_t ldb, int N, float* C, int64_t ldc, hipStream_t s);
 hipError_t launch_zero_window_rows(const SpmmPlanDev& p, int nwin, float* C, int64_t ldc, int N, hipStream_t s);

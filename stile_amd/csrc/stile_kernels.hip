@@ -14,124 +14,14 @@
 //                    products + dense 16x16 blocks on MFMA with sampled
 //                    scatter (my_fuse_formats.py:2263-2317, 2324-2415,
 //                    2519-2560)
-#include "stile_internal.h"
-
-#include <hip/hip_bf16.h>
+#include "stile_device.h"
 
 #include <algorithm>
 #include <atomic>
-#include <type_traits>
 #include <cstdlib>
 #include <cstring>
 
 namespace stile {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ float4 ld4(const float* p) {
-  return *reinterpret_cast<const float4*>(p);
-}
-__device__ __forceinline__ void st4(float* p, float4 v) {
-  *reinterpret_cast<float4*>(p) = v;
-}
-__device__ __forceinline__ float comp(const float4& v, int t) {
-  return t == 0 ? v.x : (t == 1 ? v.y : (t == 2 ? v.z : v.w));
-}
-
-// Neumaier compensated accumulation: s + c carries the sum of every x added.
-// Contraction is off so (s - t) + x is evaluated as written.
-__device__ __forceinline__ void neu_add(float& s, float& c, float x) {
-#pragma clang fp contract(off)
-  float t = s + x;
-  if (fabsf(s) >= fabsf(x))
-    c += (s - t) + x;
-  else
-    c += (x - t) + s;
-  s = t;
-}
-
-// Elements of B: FP32, BF16 or FP16.  load_b4 returns four consecutive
-// columns of row k starting at column col as FP32 (exact for the 16-bit
-// types); columns at or beyond N read as 0.  vec: B rows are aligned for one
-// vector load of four elements (16 bytes FP32, 8 bytes 16-bit) and N % 4 == 0.
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ float bf16_lo(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
-__device__ __forceinline__ float bf16_hi(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
-
-template <typename TB>
-__device__ __forceinline__ float4 cvt4(uint2 w) {
-  if constexpr (std::is_same<TB, __bf16>::value) {
-    return make_float4(bf16_lo(w.x), bf16_hi(w.x), bf16_lo(w.y), bf16_hi(w.y));
-  } else {
-    const f16x2 a = __builtin_bit_cast(f16x2, w.x), b = __builtin_bit_cast(f16x2, w.y);
-    return make_float4((float)a[0], (float)a[1], (float)b[0], (float)b[1]);
-  }
-}
-
-// B[k][col .. col + 3] as float4, zero at or beyond N.  vec (N % 4 == 0,
-// rows aligned): one unconditional load from a column clamped into the row
-// and a select after it.  (A load under an exec mask leaves its registers
-// partly unwritten, and the compiler then waits for every load in flight
-// before it reuses them: in a loop of gathers that serialises the gathers.)
-template <typename TB>
-__device__ __forceinline__ float4 load_b4(const TB* __restrict__ B, int64_t ldb, int k, int col, int N, bool vec) {
-  const TB* p = B + (int64_t)k * ldb + col;
-  if (vec) {
-    const TB* q = B + (int64_t)k * ldb + min(col, N - 4);
-    float4 r;
-    if constexpr (std::is_same<TB, float>::value)
-      r = ld4(q);
-    else
-      r = cvt4<TB>(*reinterpret_cast<const uint2*>(q));
-    return col < N ? r : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  float4 r;
-  r.x = col < N ? (float)p[0] : 0.f;
-  r.y = col + 1 < N ? (float)p[1] : 0.f;
-  r.z = col + 2 < N ? (float)p[2] : 0.f;
-  r.w = col + 3 < N ? (float)p[3] : 0.f;
-  return r;
-}
-
-// f(std::true_type) when vec, else f(std::false_type): the row gathers of
-// the sparse kernels see vec as a constant, so the 16-byte and the
-// per-element paths of load_b4 are not merged into one loop, where the
-// per-element path's masked loads make every gather wait for the ones
-// before it.
-template <typename F>
-__device__ __forceinline__ void with_vec(bool vec, F&& f) {
-  if (vec)
-    f(std::true_type{});
-  else
-    f(std::false_type{});
-}
-
-// NT: non-temporal store (streamed past the caches; for rows nothing reads
-// back soon).
-template <bool NT = false>
-__device__ __forceinline__ void store_c4(float* __restrict__ C, int64_t ldc,
-                                         int row, int col, int N, bool vec,
-                                         float4 v) {
-  float* p = C + (int64_t)row * ldc + col;
-  if (vec) {
-    if (col < N) {
-      if constexpr (NT) {
-        typedef float f32v4 __attribute__((ext_vector_type(4)));
-        __builtin_nontemporal_store(f32v4{v.x, v.y, v.z, v.w}, reinterpret_cast<f32v4*>(p));
-      } else {
-        st4(p, v);
-      }
-    }
-    return;
-  }
-  if (col < N) p[0] = v.x;
-  if (col + 1 < N) p[1] = v.y;
-  if (col + 2 < N) p[2] = v.z;
-  if (col + 3 < N) p[3] = v.w;
-}
 
 // ---------------------------------------------------------------------------
 // Plain CSR SpMM.  A segment of LPR lanes owns one row and CPL groups of
@@ -862,31 +752,7 @@ __global__ __launch_bounds__(256) void hyb_spmm_sparse_split_kernel(SpmmPlanDev 
 // (k-slot order within each chunk).
 // ---------------------------------------------------------------------------
 
-__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
-  const uint16_t a = __builtin_bit_cast(uint16_t, (__bf16)lo);
-  const uint16_t b = __builtin_bit_cast(uint16_t, (__bf16)hi);
-  return (uint32_t)a | ((uint32_t)b << 16);
-}
-
-__device__ __forceinline__ uint32_t half_sel(uint32_t x, uint32_t y, int hi) {
-  // (x.lo, y.lo) or (x.hi, y.hi) as one packed pair: one v_perm_b32, whose
-  // selector bytes 0-3 pick bytes of its second operand (x), 4-7 of its
-  // first (y)
-  return __builtin_amdgcn_perm(y, x, hi ? 0x07060302u : 0x05040100u);
-}
-
 constexpr int kLdsThreads = 1024;
-
-typedef short i16x4 __attribute__((ext_vector_type(4)));
-typedef short i16x8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) unsigned char lds_u8;
-typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-typedef __attribute__((address_space(3))) uint16_t lds_u16;
-typedef __attribute__((address_space(3))) uint32_t lds_u32;
-
-__device__ __forceinline__ i16x4 lds_tr_read(lds_u8* p) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_i16x4*>(p));
-}
 
 // Stage B[koff : koff + ksz, n0 : n0 + 64] into the LDS rows.  Consecutive
 // threads take consecutive 16-byte pieces of the block, so every load
@@ -1813,216 +1679,6 @@ hipError_t launch_row_softmax(int M, const int32_t* indptr, const float* in, flo
   const int64_t waves = M;
   hipLaunchKernelGGL(row_softmax_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, M, indptr, in, out,
                      scale);
-  return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// Fused sparse attention: out = softmax(scale * Q K^T on the mask) V for BF16
-// Q, K, V (rows x 64, leading dimension ld), FP32 out, over a plan built by
-// stile_plan_create_attention (block-diagonal masks; tc_mask marks the mask
-// entries among each chunk's k-slots).  One wave per window of 16 query rows;
-// lane l holds query q = l & 15 and lane group g = l >> 4.
-//
-// Per chunk of 32 key columns (k-slots):
-//   S^T = K Q^T as two 16x16 tiles (keys x queries), two v_mfma_f32_16x16x32_
-//     bf16 each over the 64 features (lane group g carries features
-//     32s + 8g .. +7 of step s for both operands, one 16-byte load each);
-//     lane (g, q) then holds S[q][slot 16T + 4g + i], i = 0..3, T = 0, 1;
-//   online softmax per query (running max m and sum l; the chunk max is
-//     reduced over the four lanes of a query with xor shuffles);
-//   O^T += V^T P^T as four d-tiles of one v_mfma_f32_16x16x32_bf16: the
-//     lane's eight probabilities are its B operand as they are (k-slot e of
-//     lane group g = slot 4g + e for e < 4, 16 + 4g + e - 4 otherwise); the
-//     V rows of the chunk go through LDS transposed (Vt[d][slot]) so the A
-//     operand is two ds_read_b64 per d-tile.
-// Sparse entries of a window row (the plan's sparse part) follow one at a
-// time: the four lanes of the query share the dot product and the update.
-// Out row r = O[r] / l[r] (0 for a row without entries).
-// ---------------------------------------------------------------------------
-constexpr int kAttD = 64;
-// Vt row stride in uint2 (4 BF16): 9, not 8, so that the eight d rows one
-// ds_write_b64 touches start on different LDS banks
-constexpr int kVtStride = 9;
-
-__global__ __launch_bounds__(256) void attention_fused_kernel(SpmmPlanDev p, const __bf16* __restrict__ Qm,
-                                                              const __bf16* __restrict__ Km,
-                                                              const __bf16* __restrict__ Vm, int64_t ld,
-                                                              float scale, float* __restrict__ out, int64_t ldo) {
-  __shared__ uint2 vt_all[4][kAttD * kVtStride];  // per wave: Vt[d][quad of slots], 4 BF16 each
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int w = blockIdx.x * 4 + wv;
-  if (w >= p.W) return;
-  uint2* vt = vt_all[wv];
-  const int q = lane & 15, g = lane >> 4;
-  const int row = p.win_rows[w * 16 + q];
-  const int64_t qrow = row >= 0 ? row : 0;  // padding query rows compute on row 0, store nothing
-  const bf16x8 qb0 = *reinterpret_cast<const bf16x8*>(Qm + qrow * ld + 8 * g);
-  const bf16x8 qb1 = *reinterpret_cast<const bf16x8*>(Qm + qrow * ld + 32 + 8 * g);
-  f32x4 acc[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, lsum = 0.f;
-  const int c0 = p.tc_ptr[w], c1 = p.tc_ptr[w + 1];
-  const int a = lane >> 3, o = lane & 7;
-  // the column ids this lane needs from a chunk: K rows of slots q and
-  // 16 + q (its A-operand rows), V rows of slots 4a + u (a = lane >> 3)
-  int ids[6];
-  auto load_ids = [&](int c) {
-    const int32_t* cc = p.tc_cols + (int64_t)c * 32;
-    ids[0] = cc[(q & 3) * 8 + (q >> 2)];
-    ids[1] = cc[(q & 3) * 8 + 4 + (q >> 2)];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) ids[2 + u] = cc[u * 8 + a];
-  };
-  // K and V of chunk c + 1 are requested before chunk c is processed (two
-  // register sets, loop unrolled by two so neither is copied); column ids run
-  // one chunk further ahead.
-  struct AttRegs {
-    bf16x8 k00, k01, k10, k11;
-    uint4 vv[4];
-    uint32_t mw;
-  };
-  auto load_regs = [&](int c, AttRegs& r) {
-    r.k00 = *reinterpret_cast<const bf16x8*>(Km + (int64_t)ids[0] * ld + 8 * g);
-    r.k01 = *reinterpret_cast<const bf16x8*>(Km + (int64_t)ids[0] * ld + 32 + 8 * g);
-    r.k10 = *reinterpret_cast<const bf16x8*>(Km + (int64_t)ids[1] * ld + 8 * g);
-    r.k11 = *reinterpret_cast<const bf16x8*>(Km + (int64_t)ids[1] * ld + 32 + 8 * g);
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      r.vv[u] = *reinterpret_cast<const uint4*>(Vm + (int64_t)ids[2 + u] * ld + 8 * o);
-    r.mw = p.tc_mask[(int64_t)c * 16 + q];
-  };
-  auto process = [&](const AttRegs& r) {
-    const bf16x8 &k00 = r.k00, &k01 = r.k01, &k10 = r.k10, &k11 = r.k11;
-    const uint4* vv = r.vv;
-    const uint32_t mw = r.mw;
-    f32x4 st0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k00, qb0, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-    st0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k01, qb1, st0, 0, 0, 0);
-    f32x4 st1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k10, qb0, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-    st1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k11, qb1, st1, 0, 0, 0);
-    // Vt[d][slot] for d = 8o + e, slots 4a .. 4a + 3
-    {
-      const uint32_t* v0 = reinterpret_cast<const uint32_t*>(&vv[0]);
-      const uint32_t* v1 = reinterpret_cast<const uint32_t*>(&vv[1]);
-      const uint32_t* v2 = reinterpret_cast<const uint32_t*>(&vv[2]);
-      const uint32_t* v3 = reinterpret_cast<const uint32_t*>(&vv[3]);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int h = e & 1, dw = e >> 1;
-        vt[(8 * o + e) * kVtStride + a] = make_uint2(half_sel(v0[dw], v1[dw], h), half_sel(v2[dw], v3[dw], h));
-      }
-    }
-    // online softmax
-    float sv[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      sv[i] = (mw >> (4 * g + i)) & 1u ? st0[i] : -INFINITY;
-      sv[4 + i] = (mw >> (16 + 4 * g + i)) & 1u ? st1[i] : -INFINITY;
-    }
-    float cm = sv[0];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) cm = fmaxf(cm, sv[i]);
-    cm = fmaxf(cm, __shfl_xor(cm, 16));
-    cm = fmaxf(cm, __shfl_xor(cm, 32));
-    const float m_new = fmaxf(m, cm);
-    const float alpha = m_new == -INFINITY ? 1.f : __expf((m - m_new) * scale);
-    uint32_t pk[4];
-    float psum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float pa = sv[2 * i] == -INFINITY ? 0.f : __expf((sv[2 * i] - m_new) * scale);
-      const float pb = sv[2 * i + 1] == -INFINITY ? 0.f : __expf((sv[2 * i + 1] - m_new) * scale);
-      pk[i] = bf16_pair(pa, pb);
-      // the sum uses the BF16-rounded probabilities the MFMA multiplies
-      psum += __builtin_bit_cast(float, pk[i] << 16) + __builtin_bit_cast(float, pk[i] & 0xffff0000u);
-    }
-    lsum = lsum * alpha + psum;
-    m = m_new;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] *= alpha;
-    // LDS writes of this wave complete before its reads below
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __builtin_amdgcn_wave_barrier();
-    const bf16x8 pb = __builtin_bit_cast(bf16x8, make_uint4(pk[0], pk[1], pk[2], pk[3]));
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int d = 16 * t + q;
-      const uint2 lo = vt[d * kVtStride + g], hi = vt[d * kVtStride + 4 + g];
-      const bf16x8 va = __builtin_bit_cast(bf16x8, make_uint4(lo.x, lo.y, hi.x, hi.y));
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb, acc[t], 0, 0, 0);
-    }
-    // reads of Vt done before the next chunk overwrites it
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __builtin_amdgcn_wave_barrier();
-    };
-  if (c0 < c1) {
-    const int last = c1 - 1;
-    AttRegs R0, R1;
-    load_ids(c0);
-    load_regs(c0, R0);
-    load_ids(min(c0 + 1, last));
-    int c = c0;
-    while (c + 2 <= c1) {
-      load_regs(min(c + 1, last), R1);
-      load_ids(min(c + 2, last));
-      process(R0);
-      ++c;
-      load_regs(min(c + 1, last), R0);
-      load_ids(min(c + 2, last));
-      process(R1);
-      ++c;
-    }
-    if (c < c1) process(R0);
-  }
-  // sparse entries of the window rows, one per step for all 16 queries
-  {
-    const int r0 = p.res_ptr[w * 16 + q], r1 = p.res_ptr[w * 16 + q + 1];
-    int n = r1 - r0;
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) n = max(n, __shfl_xor(n, off));
-    for (int j = 0; j < n; ++j) {
-      const bool on = r0 + j < r1;
-      const int col = on ? p.res_cols[r0 + j] : 0;
-      const bf16x8 ka = *reinterpret_cast<const bf16x8*>(Km + (int64_t)col * ld + 8 * g);
-      const bf16x8 kb = *reinterpret_cast<const bf16x8*>(Km + (int64_t)col * ld + 32 + 8 * g);
-      float dot = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) dot += (float)qb0[e] * (float)ka[e] + (float)qb1[e] * (float)kb[e];
-      dot += __shfl_xor(dot, 16);
-      dot += __shfl_xor(dot, 32);
-      const float sval = on ? dot : -INFINITY;
-      const float m_new = fmaxf(m, sval);
-      const float alpha = m_new == -INFINITY ? 1.f : __expf((m - m_new) * scale);
-      const float pr = sval == -INFINITY ? 0.f : __expf((sval - m_new) * scale);
-      const float prb = __builtin_bit_cast(float, bf16_pair(pr, 0.f) << 16);
-      lsum = lsum * alpha + (g == 0 ? prb : 0.f);
-      m = m_new;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const uint2 vr = *reinterpret_cast<const uint2*>(Vm + (int64_t)col * ld + 16 * t + 4 * g);
-        acc[t][0] = acc[t][0] * alpha + prb * __builtin_bit_cast(float, vr.x << 16);
-        acc[t][1] = acc[t][1] * alpha + prb * __builtin_bit_cast(float, vr.x & 0xffff0000u);
-        acc[t][2] = acc[t][2] * alpha + prb * __builtin_bit_cast(float, vr.y << 16);
-        acc[t][3] = acc[t][3] * alpha + prb * __builtin_bit_cast(float, vr.y & 0xffff0000u);
-      }
-    }
-  }
-  float ltot = lsum + __shfl_xor(lsum, 16);
-  ltot += __shfl_xor(ltot, 32);
-  if (row < 0) return;
-  const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-    st4(out + (int64_t)row * ldo + 16 * t + 4 * g,
-        make_float4(acc[t][0] * inv, acc[t][1] * inv, acc[t][2] * inv, acc[t][3] * inv));
-}
-
-hipError_t launch_attention(const SpmmPlanDev& p, const void* Q, const void* K, const void* V, int64_t ld,
-                            float scale, float* out, int64_t ldo, hipStream_t s) {
-  if (p.W == 0) return hipSuccess;
-  hipLaunchKernelGGL(attention_fused_kernel, dim3((unsigned)((p.W + 3) / 4)), dim3(256), 0, s, p,
-                     static_cast<const __bf16*>(Q), static_cast<const __bf16*>(K), static_cast<const __bf16*>(V),
-                     ld, scale, out, ldo);
   return hipGetLastError();
 }
 

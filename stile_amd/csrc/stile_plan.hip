@@ -42,6 +42,7 @@ struct StilePlan {
   const int32_t* res_ids = nullptr;
   int64_t n_sp = 0;
   const int32_t* sp_ids = nullptr;
+  stile::AttOrder att{};  // attention plans
   // per-XCD item ranges of the B-stationary kernel (spmm.lds_xcd_host)
   std::vector<int32_t> lds_xcd;
 };
@@ -617,6 +618,36 @@ std::vector<std::array<int32_t, 32>> place_scatter(const std::vector<ScatEnt>& s
   return out;
 }
 
+// Launch order of the fused attention kernel (AttOrder): windows by first
+// row, cut into kXcds ranges where the running cost is nearest to x / kXcds of
+// the total.  A window costs a fixed part, its chunks and, per step of the
+// sparse part (kAttSparseStep entries of each row), about two chunks (a step
+// waits for its own K and V rows, a chunk's are requested one chunk ahead).
+constexpr int32_t kAttSparseStep = 4;
+
+void attention_order(const std::vector<int32_t>& win_rows, const std::vector<int32_t>& tc_ptr,
+                     const std::vector<int32_t>& res_ptr, std::vector<int32_t>& win,
+                     int32_t (&start)[stile::kXcds + 1]) {
+  const int32_t W = (int32_t)(win_rows.size() / 16);
+  std::vector<int32_t> first(W, INT32_MAX);
+  std::vector<int64_t> cost(W, 2);
+  for (int32_t w = 0; w < W; ++w) {
+    int32_t longest = 0;
+    for (int r = 0; r < 16; ++r) {
+      const int32_t row = win_rows[(size_t)w * 16 + r];
+      if (row >= 0) first[w] = std::min(first[w], row);
+      longest = std::max(longest, res_ptr[(size_t)w * 16 + r + 1] - res_ptr[(size_t)w * 16 + r]);
+    }
+    cost[w] += tc_ptr[w + 1] - tc_ptr[w] + (longest + kAttSparseStep - 1) / kAttSparseStep * 2;
+  }
+  win.resize(W);
+  for (int32_t w = 0; w < W; ++w) win[w] = w;
+  std::stable_sort(win.begin(), win.end(), [&](int32_t a, int32_t b) { return first[a] < first[b]; });
+  std::vector<int64_t> by_order(W);
+  for (int32_t i = 0; i < W; ++i) by_order[i] = cost[win[i]];
+  lds_xcd_split(by_order, 1, start);
+}
+
 int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan** out) {
   const int32_t W = (int32_t)(bd.win_rows.size() / 16);
   bd.win_scat.assign(W, {});
@@ -959,7 +990,8 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   const size_t o_tcvals = lay.add(tc_vals.size());
   const size_t o_scale = lay.add(tc_scale.size() * 4);
   const size_t o_resptr = lay.add(res_ptr.size() * 4);
-  const size_t o_rescols = lay.add(res_cols.size() * 4);
+  // (16 bytes past the end: the attention kernel reads a row's ids four at a time)
+  const size_t o_rescols = lay.add(res_cols.size() * 4 + 16);
   const size_t o_resvals = lay.add(res_vals.size() * 4);
   // the fix-up kernel's piece order (see SpmmPlanDev::piece_exec)
   std::vector<int32_t> piece_exec(piece_row.size());
@@ -1000,6 +1032,10 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
     if (run) win_r0[w] = r0;
   }
   const size_t o_r0 = lay.add(win_r0.size() * 4);
+  std::vector<int32_t> att_win;
+  stile::AttOrder att{};
+  if (bd.want_mask) attention_order(bd.win_rows, tc_ptr, res_ptr, att_win, att.start);
+  const size_t o_att = lay.add(att_win.size() * 4);
   HostBlob blob;
   blob.data.assign(lay.bytes, 0);
   blob.put(o_rows, bd.win_rows.data(), bd.win_rows.size() * 4);
@@ -1031,6 +1067,7 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   blob.put(o_spids, sp_ids.data(), sp_ids.size() * 4);
   blob.put(o_kind, tc_kind.data(), tc_kind.size() * 4);
   blob.put(o_r0, win_r0.data(), win_r0.size() * 4);
+  blob.put(o_att, att_win.data(), att_win.size() * 4);
 
   StilePlan* plan = new (std::nothrow) StilePlan();
   if (!plan) return fail(STILE_E_NOMEM, "host allocation of plan");
@@ -1078,6 +1115,8 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   d.sp_ent = sp_off.empty() ? nullptr : dptr<int2>(plan, o_spent);
   d.tc_kind = tc_kind.empty() ? nullptr : dptr<uint32_t>(plan, o_kind);
   d.win_r0 = win_r0.empty() ? nullptr : dptr<int32_t>(plan, o_r0);
+  plan->att = att;
+  plan->att.win = att_win.empty() ? nullptr : dptr<int32_t>(plan, o_att);
   d.opt_kernel = 0;
   d.opt_lds_list = -1;
   d.opt_lds_xcd = 1;
@@ -1466,7 +1505,7 @@ int stile_attention_run(const StilePlan* plan, const void* Q, const void* K, con
   if ((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V)) & 15 ||
       reinterpret_cast<uintptr_t>(out) & 15)
     return fail(STILE_E_INVALID, "Q, K, V and out must be 16-byte aligned");
-  hipError_t e = stile::launch_attention(plan->spmm, Q, K, V, ld, scale, out, ldo, (hipStream_t)stream);
+  hipError_t e = stile::launch_attention(plan->spmm, plan->att, Q, K, V, ld, scale, out, ldo, (hipStream_t)stream);
   return e == hipSuccess ? STILE_OK : hip_fail(e, "attention launch");
 }
 
