@@ -18,6 +18,10 @@ constexpr int kHubNnz = 4096;
 // mode: stores to a workspace, summed in piece order by a reduce kernel).
 constexpr int kSplitNnz = 256;
 
+// Entries of padding (column 0, value 0) behind res_cols and res_vals, for
+// kernels that read a row's entries a few at a time.
+constexpr int kRowPad = 16;
+
 // Value id of an A element that a value refresh leaves as it is (the row
 // half of a scatter chunk's k-slot word).
 constexpr int32_t kKeepId = -2;
@@ -131,6 +135,11 @@ struct SpmmPlanDev {
   const int32_t* res_cols;
   const float* res_vals;
   int32_t nnz_sparse_only;   // sparse nonzeros in windows [W_tc, W)
+  // wave tasks of the sparse-only windows' rows (hyb_spmm_rows_kernel):
+  // consecutive slots [x, y), bit 31 of y set for a row of more than kHubNnz
+  // entries
+  int32_t n_row_tasks;
+  const int2* row_tasks;
   int32_t n_mix;             // slots of dense windows with a sparse part
   const int32_t* mix_slot;   // [n_mix]
   const uint32_t* tc_mask;   // [nchunks][16] entry bits (attention plans), else nullptr
@@ -199,6 +208,17 @@ hipError_t launch_hyb_spmm(const SpmmPlanDev& p, int b_dtype, const void* B, int
                            int N, float* C, int64_t ldc, bool deterministic, float* ws, hipStream_t s);
 // Floats of workspace the deterministic mode needs at width N.
 int64_t spmm_workspace_floats(const SpmmPlanDev& p, int N);
+// Rows of the sparse-only windows, and pieces [pc0, pc1) of long rows (added
+// to C, or stored to ws).  vec: N % 4 == 0, B and C aligned for four columns.
+template <typename TB>
+hipError_t launch_sparse_rows(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc, bool vec,
+                              hipStream_t s);
+template <typename TB>
+hipError_t launch_sparse_pieces(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc,
+                                bool vec, int pc0, int pc1, float* ws, hipStream_t s);
+// Deterministic mode: split rows [sr0, nsrows) += their pieces in ws.
+hipError_t launch_piece_reduce(const SpmmPlanDev& p, int N, float* C, int64_t ldc, bool vec, int sr0, const float* ws,
+                               hipStream_t s);
 hipError_t launch_hyb_sddmm(const SddmmPlanDev& p, const float* X,
                             int64_t ldx, const float* Y, int64_t ldy, int Kf,
                             float* out, hipStream_t s);

@@ -381,18 +381,6 @@ __device__ __forceinline__ void add_slot(const SpmmPlanDev& p, const TB* __restr
   store_c4(C, ldc, row, col, N, vec, make_float4(c.x + s.x, c.y + s.y, c.z + s.z, c.w + s.w));
 }
 
-// One slot (sparse-only windows, one row per lane group).
-template <typename TB>
-__device__ __forceinline__ void finish_slot(const SpmmPlanDev& p, const TB* __restrict__ B, int64_t ldb,
-                                            int N, float* __restrict__ C, int64_t ldc, int col, bool vec,
-                                            int slot) {
-  const int row = p.win_rows[slot];
-  const int r0 = p.res_ptr[slot], rend = p.res_ptr[slot + 1];
-  const int r1 = min(rend, r0 + kSplitNnz);
-  const float4 s = sparse_row_sum<kSparseDepth>(p, B, ldb, N, col, vec, r0, r1, rend - r0 > kHubNnz);
-  if (row >= 0) store_c4(C, ldc, row, col, N, vec, s);
-}
-
 template <int MODE>
 __device__ __forceinline__ void mfma_chunk(const SpmmPlanDev& p, int64_t c, int lane, const float4 (&b)[8],
                                            f32x4 (&acc)[4]) {
@@ -606,47 +594,25 @@ __global__ __launch_bounds__(256) void hyb_spmm_part_reduce_kernel(SpmmPlanDev p
     if (sr.row[i] >= 0) store_c4(C, ldc, sr.row[i], col, N, vec, acc[i]);
 }
 
-// Sparse parts, one row per lane group: first the n_mix slots of dense
-// windows (four per wave and 64 columns, added to the stored dense rows;
-// n_mix is 0 when the B-stationary kernel adds them itself), then the
-// sparse-only windows [W_tc, W) (four waves per window and 64 columns).  A
-// kernel of its own so that its small register footprint sets its occupancy
-// (gathers in flight per CU), not the dense path's.
-// so_waves: waves for the sparse-only windows (0 when hyb_spmm_sparse_split_kernel
-// stores those rows instead).  Waves go column chunk by column chunk (all of a
-// part's waves for columns 0..63, then 64..127, ...), so that the B rows the
-// grid gathers at one time are one 64-column slice of B: on a 1 M-row graph
-// with N = 128 that slice is 256 MB instead of B's 512 MB (GCN scale-20 SpMM
-// 2.34 -> 2.26 ms with the same order in the fix-up kernel).
+// Sparse parts of the dense windows' rows after the streaming kernel, one row
+// per lane group: the n_mix slots of dense windows, four per wave and 64
+// columns, added to the stored dense rows.  Waves go column chunk by column
+// chunk.
 // (256, 7): 71 VGPRs, no spills, 7 waves per SIMD instead of 6; the row
-// gathers are latency-bound (GCN scale-20 SpMM 2.42 -> 2.34 ms).
+// gathers are latency-bound.
 template <typename TB>
 __global__ __launch_bounds__(256, 7) void hyb_spmm_sparse_kernel(SpmmPlanDev p, const TB* __restrict__ B,
                                                               int64_t ldb, int N, float* __restrict__ C,
-                                                              int64_t ldc, int nC, bool vec, int n_mix,
-                                                              int64_t so_waves) {
+                                                              int64_t ldc, int nC, bool vec, int n_mix) {
   const int lane = threadIdx.x & 63;
   const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int64_t mix_waves = (int64_t)((n_mix + 3) / 4) * nC;
-  if (wave < mix_waves) {
-    const int64_t per = (n_mix + 3) / 4;
-    const int cch = (int)(wave / per);
-    const int q = (int)(wave - cch * per);
-    const int col = cch * 64 + 4 * (lane & 15);
-    const int m = q * 4 + (lane >> 4);
-    if (m < n_mix) with_vec(vec, [&](auto V) { add_slot(p, B, ldb, N, C, ldc, col, V, p.mix_slot[m]); });
-    return;
-  }
-  const int64_t idx = wave - mix_waves;
-  if (idx >= so_waves) return;
-  const int64_t per = so_waves / nC;
-  const int cch = (int)(idx / per);
-  const int64_t rr = idx - cch * per;
-  const int w = p.W_tc + (int)(rr >> 2);
-  const int quarter = (int)(rr & 3);
-  const int n0 = cch * 64;
-  const int col = n0 + 4 * (lane & 15);
-  with_vec(vec, [&](auto V) { finish_slot(p, B, ldb, N, C, ldc, col, V, w * 16 + quarter * 4 + (lane >> 4)); });
+  const int64_t per = (n_mix + 3) / 4;
+  const int cch = (int)(wave / per);
+  if (cch >= nC) return;
+  const int q = (int)(wave - cch * per);
+  const int col = cch * 64 + 4 * (lane & 15);
+  const int m = q * 4 + (lane >> 4);
+  if (m < n_mix) with_vec(vec, [&](auto V) { add_slot(p, B, ldb, N, C, ldc, col, V, p.mix_slot[m]); });
 }
 
 // Sparse-only rows for launches with too few rows to fill the GPU at one row
@@ -1194,96 +1160,6 @@ __global__ __launch_bounds__(kLdsThreads) void hyb_spmm_lds_bf16_kernel(SpmmPlan
   }
 }
 
-// Remaining pieces of long sparse rows, execution slots [pc0, pc1) (piece
-// p.piece_exec[slot], ordered by first column so that pieces of different
-// rows gathering the same B rows run together), column chunk by column chunk
-// as in hyb_spmm_sparse_kernel: lane group g of
-// the wave takes nonzeros q = beg + g, beg + g + 4, ...; the four partial
-// float4 are reduced across groups and added to C with atomicAdd (C already
-// holds the window pass's value of the row), or, with ws (deterministic
-// mode), stored to ws[piece][N] for hyb_spmm_piece_reduce_kernel.
-template <typename TB>
-__global__ __launch_bounds__(256) void hyb_spmm_fixup_kernel(SpmmPlanDev p, const TB* __restrict__ B,
-                                                             int64_t ldb, int N, float* __restrict__ C,
-                                                             int64_t ldc, int nC, bool vec, int pc0, int pc1,
-                                                             float* __restrict__ ws) {
-  const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  const int npc = pc1 - pc0;
-  const int cch = wave / npc;
-  if (cch >= nC) return;
-  const int pe = pc0 + (wave - cch * npc);
-  const int pc = p.piece_exec[pe];
-  const int n0 = cch * 64;
-  const int lane = threadIdx.x & 63;
-  const int g = lane >> 4;
-  const int col = n0 + 4 * (lane & 15);
-  const int beg = p.piece_beg[pc], end = p.piece_end[pc];
-  with_vec(vec, [&](auto V) {
-  float4 s = make_float4(0.f, 0.f, 0.f, 0.f), cc = make_float4(0.f, 0.f, 0.f, 0.f);
-  // eight gathers in flight per lane group (positions past the end read the
-  // piece's last entry with weight 0)
-  for (int q0 = beg + g; q0 < end; q0 += 32) {
-    int k[8];
-    float v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int q = q0 + 4 * i;
-      const int qc = min(q, end - 1);
-      k[i] = p.res_cols[qc];
-      v[i] = q < end ? p.res_vals[qc] : 0.f;
-    }
-    float4 b[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) b[i] = load_b4(B, ldb, k[i], col, N, V);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      neu_add(s.x, cc.x, v[i] * b[i].x);
-      neu_add(s.y, cc.y, v[i] * b[i].y);
-      neu_add(s.z, cc.z, v[i] * b[i].z);
-      neu_add(s.w, cc.w, v[i] * b[i].w);
-    }
-  }
-  s.x += cc.x; s.y += cc.y; s.z += cc.z; s.w += cc.w;
-#pragma unroll
-  for (int off = 16; off <= 32; off <<= 1) {
-    s.x += __shfl_xor(s.x, off);
-    s.y += __shfl_xor(s.y, off);
-    s.z += __shfl_xor(s.z, off);
-    s.w += __shfl_xor(s.w, off);
-  }
-  if (g != 0) return;
-  if (ws) {
-    store_c4(ws, N, pc, col, N, V, s);
-    return;
-  }
-  float* cp = C + (int64_t)p.piece_row[pc] * ldc + col;
-  if (col < N) atomicAdd(cp, s.x);
-  if (col + 1 < N) atomicAdd(cp + 1, s.y);
-  if (col + 2 < N) atomicAdd(cp + 2, s.z);
-  if (col + 3 < N) atomicAdd(cp + 3, s.w);
-  });
-}
-
-// Deterministic mode: C[row] += the row's pieces in piece order, for split
-// rows [sr0, sr1).  One 16-lane group per (split row, 64 columns); C[row] is
-// read and written by that group alone.
-__global__ __launch_bounds__(256) void hyb_spmm_piece_reduce_kernel(SpmmPlanDev p, int N, float* __restrict__ C,
-                                                                    int64_t ldc, int nC, bool vec, int sr0,
-                                                                    int sr1, const float* __restrict__ ws) {
-  const int64_t task = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
-  const int r = sr0 + (int)(task / nC);
-  if (r >= sr1) return;
-  const int col = (int)(task - (int64_t)(r - sr0) * nC) * 64 + 4 * (threadIdx.x & 15);
-  const int row = p.srow_row[r];
-  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int q = p.srow_p0[r]; q < p.srow_p1[r]; ++q) {
-    const float4 v = load_b4(ws, N, q, col, N, vec);
-    s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-  }
-  const float4 c = load_b4(C, ldc, row, col, N, vec);
-  store_c4(C, ldc, row, col, N, vec, make_float4(c.x + s.x, c.y + s.y, c.z + s.z, c.w + s.w));
-}
-
 template <bool kLoop, typename TB>
 static void set_lds_bytes(int bytes) {
   for (const void* f : {reinterpret_cast<const void*>(hyb_spmm_lds_bf16_kernel<kLoop, TB, false, false>),
@@ -1443,14 +1319,14 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
       if (e != hipSuccess) return e;
     }
   }
-  // Sparse-only rows (unless folded) one per lane group, or, when that
-  // leaves fewer than 16 waves per CU for rows of 8 or more nonzeros on
-  // average, one per wave; before them, unless the LDS kernel added them,
-  // the sparse parts of the dense windows' rows.
+  // Sparse-only rows (unless folded) by wave tasks, or, when there are fewer
+  // than 16,384 (row, 64 columns) of 8 or more nonzeros on average, one of those
+  // per wave with all its gathers in flight at once; then, unless the LDS kernel
+  // added them, the sparse parts of the dense windows' rows.
   const int n_mix = lds ? 0 : p.n_mix;
   const int64_t so_left = fold ? 0 : so_rows;
   const bool split = so_left > 0 && so_left * nC / 4 < 4096 && p.nnz_sparse_only >= 8 * so_left;
-  const int64_t sparse_waves = (int64_t)((n_mix + 3) / 4) * nC + (split ? 0 : so_left * nC / 4);
+  const int64_t sparse_waves = (int64_t)((n_mix + 3) / 4) * nC;
   if (split) {
     const int64_t blocks = (so_rows * nC + 3) / 4;
     hipLaunchKernelGGL(hyb_spmm_sparse_split_kernel<TB>, dim3((unsigned)blocks), dim3(256), 0, s, p, B, ldb, N, C,
@@ -1458,11 +1334,15 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
+  if (so_left > 0 && !split) {
+    hipError_t e = launch_sparse_rows(p, B, ldb, N, C, ldc, vec, s);
+    if (e != hipSuccess) return e;
+  }
   if (sparse_waves > 0) {
     const int64_t blocks = (sparse_waves + 3) / 4;
     if (blocks > INT32_MAX) return hipErrorInvalidValue;
     hipLaunchKernelGGL(hyb_spmm_sparse_kernel<TB>, dim3((unsigned)blocks), dim3(256), 0, s, p, B, ldb, N, C, ldc,
-                       nC, vec, n_mix, split ? (int64_t)0 : so_left * nC / 4);
+                       nC, vec, n_mix);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
@@ -1470,20 +1350,11 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
   // only the sparse-only rows' pieces remain after it.
   const int pc0 = lds ? p.npieces_dense : 0;
   if (p.npieces > pc0) {
-    const int64_t fw = (int64_t)(p.npieces - pc0) * nC;
-    hipLaunchKernelGGL(hyb_spmm_fixup_kernel<TB>, dim3((unsigned)((fw + 3) / 4)), dim3(256), 0, s, p, B, ldb, N,
-                       C, ldc, nC, vec, pc0, p.npieces, ws_pieces);
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_sparse_pieces(p, B, ldb, N, C, ldc, vec, pc0, p.npieces, ws_pieces, s);
     if (e != hipSuccess) return e;
     if (det) {
-      const int sr0 = lds ? p.nsrows_dense : 0;
-      const int64_t tasks = (int64_t)(p.nsrows - sr0) * nC;
-      if (tasks > 0) {
-        hipLaunchKernelGGL(hyb_spmm_piece_reduce_kernel, dim3((unsigned)((tasks + 15) / 16)), dim3(256), 0, s, p,
-                           N, C, ldc, nC, vec, sr0, p.nsrows, ws_pieces);
-        e = hipGetLastError();
-        if (e != hipSuccess) return e;
-      }
+      e = launch_piece_reduce(p, N, C, ldc, vec, lds ? p.nsrows_dense : 0, ws_pieces, s);
+      if (e != hipSuccess) return e;
     }
   }
   return hipSuccess;

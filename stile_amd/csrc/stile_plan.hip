@@ -648,6 +648,38 @@ void attention_order(const std::vector<int32_t>& win_rows, const std::vector<int
   lds_xcd_split(by_order, 1, start);
 }
 
+// Wave tasks over the slots [s0, s1) (SpmmPlanDev::row_tasks): consecutive
+// slots until they hold `target` entries, a row of more than kSplitNnz alone.
+// 64 entries a task hide the latencies at its start and end; a plan with fewer
+// than 8,192 such tasks (eight waves per SIMD) takes smaller ones, down to 16
+// entries.  Tasks of 128 entries and more run first, so that none of them
+// starts when the others are done.
+std::vector<int32_t> sparse_row_tasks(const std::vector<int64_t>& ptr, int64_t s0, int64_t s1) {
+  const int64_t target = std::min<int64_t>(64, std::max<int64_t>(16, (ptr[s1] - ptr[s0]) / 8192));
+  constexpr int64_t kMaxSlots = 64, kLong = 128;
+  std::vector<std::array<int32_t, 2>> tasks;
+  int64_t a = s0;
+  for (int64_t s = s0; s < s1; ++s) {
+    const int64_t len = ptr[s + 1] - ptr[s];
+    if (len > stile::kSplitNnz) {
+      if (s > a) tasks.push_back({(int32_t)a, (int32_t)s});
+      tasks.push_back({(int32_t)s, (int32_t)((uint32_t)(s + 1) | (len > stile::kHubNnz ? 0x80000000u : 0u))});
+      a = s + 1;
+    } else if (ptr[s + 1] - ptr[a] >= target || s + 1 - a >= kMaxSlots) {
+      tasks.push_back({(int32_t)a, (int32_t)(s + 1)});
+      a = s + 1;
+    }
+  }
+  if (a < s1) tasks.push_back({(int32_t)a, (int32_t)s1});
+  std::stable_partition(tasks.begin(), tasks.end(), [&](const std::array<int32_t, 2>& t) {
+    return ptr[t[1] & 0x7fffffff] - ptr[t[0]] >= kLong;
+  });
+  std::vector<int32_t> out;
+  out.reserve(tasks.size() * 2);
+  for (const auto& t : tasks) out.insert(out.end(), t.begin(), t.end());
+  return out;
+}
+
 int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan** out) {
   const int32_t W = (int32_t)(bd.win_rows.size() / 16);
   bd.win_scat.assign(W, {});
@@ -812,6 +844,8 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
       nsrows_dense = (int32_t)srow_row.size();
     }
   }
+
+  const std::vector<int32_t> row_tasks = sparse_row_tasks(cnt, (int64_t)W_tc * 16, (int64_t)W * 16);
 
   if (lds_ok)
     for (int32_t w = 0; w < W_tc; ++w) order_chunk_slots(bd.win_cols[w], bd.inst_cols[window_matrix(bd, w)]);
@@ -990,9 +1024,8 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   const size_t o_tcvals = lay.add(tc_vals.size());
   const size_t o_scale = lay.add(tc_scale.size() * 4);
   const size_t o_resptr = lay.add(res_ptr.size() * 4);
-  // (16 bytes past the end: the attention kernel reads a row's ids four at a time)
-  const size_t o_rescols = lay.add(res_cols.size() * 4 + 16);
-  const size_t o_resvals = lay.add(res_vals.size() * 4);
+  const size_t o_rescols = lay.add((res_cols.size() + stile::kRowPad) * 4);
+  const size_t o_resvals = lay.add((res_vals.size() + stile::kRowPad) * 4);
   // the fix-up kernel's piece order (see SpmmPlanDev::piece_exec)
   std::vector<int32_t> piece_exec(piece_row.size());
   for (size_t q = 0; q < piece_exec.size(); ++q) piece_exec[q] = (int32_t)q;
@@ -1035,6 +1068,7 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   std::vector<int32_t> att_win;
   stile::AttOrder att{};
   if (bd.want_mask) attention_order(bd.win_rows, tc_ptr, res_ptr, att_win, att.start);
+  const size_t o_rtask = lay.add(row_tasks.size() * 4);
   const size_t o_att = lay.add(att_win.size() * 4);
   HostBlob blob;
   blob.data.assign(lay.bytes, 0);
@@ -1067,6 +1101,7 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   blob.put(o_spids, sp_ids.data(), sp_ids.size() * 4);
   blob.put(o_kind, tc_kind.data(), tc_kind.size() * 4);
   blob.put(o_r0, win_r0.data(), win_r0.size() * 4);
+  blob.put(o_rtask, row_tasks.data(), row_tasks.size() * 4);
   blob.put(o_att, att_win.data(), att_win.size() * 4);
 
   StilePlan* plan = new (std::nothrow) StilePlan();
@@ -1090,6 +1125,8 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   d.part_win = dptr<int32_t>(plan, o_pwin);
   d.part_c0 = dptr<int32_t>(plan, o_pc0);
   d.part_c1 = dptr<int32_t>(plan, o_pc1);
+  d.n_row_tasks = (int32_t)(row_tasks.size() / 2);
+  d.row_tasks = dptr<int2>(plan, o_rtask);
   d.n_mix = (int32_t)mix_slot.size();
   d.mix_slot = dptr<int32_t>(plan, o_mix);
   d.tc_mask = tc_mask.empty() ? nullptr : dptr<uint32_t>(plan, o_mask);
