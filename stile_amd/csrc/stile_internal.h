@@ -20,17 +20,27 @@ constexpr int kSplitNnz = 256;
 
 // Entries of padding (column 0, value 0) behind res_cols and res_vals, for
 // kernels that read a row's entries a few at a time.
-constexpr int kRowPad = 16;
+constexpr int kRowPad = 32;
+
+// Flags of a wave task of the sparse rows (SpmmPlanDev::row_tasks).
+constexpr int32_t kTaskSlots = 0x3fffffff, kTaskAdd = 0x40000000, kTaskHub = (int32_t)0x80000000;
 
 // Value id of an A element that a value refresh leaves as it is (the row
 // half of a scatter chunk's k-slot word).
 constexpr int32_t kKeepId = -2;
-// Windows with more than kBigChunks dense chunks are "big": the streaming
-// kernel gives each (big window, 64 columns) a workgroup of kBigWaves waves,
-// each wave a contiguous share of the chunks, and sums the partial results
-// through LDS in wave order.
-constexpr int kBigChunks = 8;
-constexpr int kBigWaves = 8;
+// The streaming kernel gives each (window, 64 columns) a workgroup, each of its
+// waves a contiguous share of the window's chunks, and sums the partial results
+// through LDS in wave order.  Windows with more than kBigChunks chunks are "big"
+// and take 32 columns a workgroup: twice the workgroups, and four chunks in
+// flight per wave instead of two, for the windows a launch waits for.
+constexpr int kBigChunks = 16;
+// Windows with more than kLongChunks chunks come first in a plan, most chunks first.
+constexpr int kLongChunks = 8;
+// Sparse parts of dense windows whose rows have at most this many entries are
+// summed by the streaming kernel's workgroup of the window (no second launch, no
+// second pass over C); longer ones by the sparse-row kernel's tasks, which are
+// balanced over the whole GPU.
+constexpr int kFoldMaxLen = 128;
 // Windows with more than kHugeChunks chunks (hub rows of power-law graphs)
 // are cut into parts of at most kHugeChunks chunks, one workgroup each, that
 // add their partial rows into C with atomicAdd (those rows are zeroed first):
@@ -81,6 +91,7 @@ struct SpmmPlanDev {
   int32_t W_tc;              // windows [0, W_tc) hold dense chunks; the rest are sparse-only
   int32_t W_big;             // windows [0, W_big) hold more than kBigChunks chunks
   int32_t W_huge;            // windows [0, W_huge) hold more than kHugeChunks chunks
+  int32_t chunks_small;      // chunks of windows [W_big, W_tc)
   int32_t n_parts;           // parts of the huge windows
   const int32_t* part_win;   // [n_parts] window of each part
   const int32_t* part_c0;    // [n_parts] chunk range of each part
@@ -135,13 +146,13 @@ struct SpmmPlanDev {
   const int32_t* res_cols;
   const float* res_vals;
   int32_t nnz_sparse_only;   // sparse nonzeros in windows [W_tc, W)
-  // wave tasks of the sparse-only windows' rows (hyb_spmm_rows_kernel):
-  // consecutive slots [x, y), bit 31 of y set for a row of more than kHubNnz
-  // entries
-  int32_t n_row_tasks;
+  // wave tasks of hyb_spmm_rows_kernel: consecutive slots [x, y & kTaskSlots)
+  // with the flags kTaskHub and kTaskAdd in y; the first n_mix_tasks are slots
+  // of dense windows, the others of sparse-only windows
+  int32_t n_row_tasks, n_mix_tasks;
   const int2* row_tasks;
   int32_t n_mix;             // slots of dense windows with a sparse part
-  const int32_t* mix_slot;   // [n_mix]
+  int32_t fold_mix;          // 1: none of them holds more than kFoldMaxLen entries
   const uint32_t* tc_mask;   // [nchunks][16] entry bits (attention plans), else nullptr
   // B-stationary work units (BF16 plans with every matrix's K <= kLdsMaxK):
   // unit = (first window, end window, first B row, B rows) of one matrix,
@@ -208,11 +219,11 @@ hipError_t launch_hyb_spmm(const SpmmPlanDev& p, int b_dtype, const void* B, int
                            int N, float* C, int64_t ldc, bool deterministic, float* ws, hipStream_t s);
 // Floats of workspace the deterministic mode needs at width N.
 int64_t spmm_workspace_floats(const SpmmPlanDev& p, int N);
-// Rows of the sparse-only windows, and pieces [pc0, pc1) of long rows (added
-// to C, or stored to ws).  vec: N % 4 == 0, B and C aligned for four columns.
+// Row tasks [t0, t1), and pieces [pc0, pc1) of long rows (added to C, or stored
+// to ws).  vec: N % 4 == 0, B and C aligned for four columns.
 template <typename TB>
 hipError_t launch_sparse_rows(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc, bool vec,
-                              hipStream_t s);
+                              int t0, int t1, hipStream_t s);
 template <typename TB>
 hipError_t launch_sparse_pieces(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc,
                                 bool vec, int pc0, int pc1, float* ws, hipStream_t s);
@@ -237,6 +248,13 @@ hipError_t launch_ell_bucket_spmm(int rows, int width, const int32_t* orow, cons
 hipError_t launch_zero_window_rows(const SpmmPlanDev& p, int nwin, float* C, int64_t ldc, int N, hipStream_t s);
 hipError_t launch_row_softmax(int M, const int32_t* indptr, const float* in, float* out, float scale,
                               hipStream_t s);
+
+// Dense windows on the streaming kernel (with their sparse parts when the plan
+// folds them, SpmmPlanDev::fold_mix).  ws: the deterministic mode's region for
+// the parts of huge windows, nullptr to add them with atomicAdd.
+template <typename TB>
+hipError_t launch_stream(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc, bool vec,
+                         float* ws, hipStream_t s);
 
 // Zero-fill kernels (used instead of hipMemsetAsync so that every *_run call
 // records only kernel nodes under HIP graph capture).

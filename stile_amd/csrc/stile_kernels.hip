@@ -226,122 +226,19 @@ hipError_t launch_csr_sddmm_f32(int M, int nnz, int Kf, const int32_t* indptr,
 // ---------------------------------------------------------------------------
 // Hybrid fused SpMM.
 //
-// One wave = (window w, 64 output columns n0..n0+63).  Lane l = 16g + j owns
-// output columns n0 + 4j .. n0 + 4j + 3 of rows 4g .. 4g+3 of the window: the
-// four 16x16 MFMA tiles t = 0..3 of the wave hold column n0 + 4j + t in MFMA
-// column j, so every B load and every C store is four consecutive columns and
-// MFMA output element (row 4g+i, column j) of tile t is exactly the lane's own
-// element.
-//
-// Dense chunk (32 k-slots): k-slot 4e + g of lane l is column tc_cols[c][g][e]
-// of A, A operand element e of lane l (the pairing of k-slots with operand
-// elements is the same for A and B, which is all the MFMA needs).
-//   BF16: one v_mfma_f32_16x16x32_bf16 per tile;
-//   FP16: one v_mfma_f32_16x16x32_f16 per tile, times the chunk's scale;
-//   FP32: eight v_mfma_f32_16x16x4_f32 per tile (MFMA e reduces k-slots
-//         4e + 0..3; lane group g supplies k-slot 4e + g).
-// Sparse part: the lane adds v * B[col][n0+4j..+3] for the FP32 nonzeros of
-// its rows (compensated when a row has more than kHubNnz).
-//
-// B is FP32, BF16 or FP16 (TB); every product and sum of the sparse part is
-// FP32 on B's exact values.
-//
 // Kernels of one run, in stream order.  Plans on the B-stationary kernel
 // (BF16 blocks, K <= kLdsMaxK): that kernel computes every dense window with
 // its sparse part, and as its tail (when they are few) the sparse-only rows;
-// otherwise the sparse kernel runs the sparse-only rows.  Other plans: the
-// streaming kernel stores the dense windows (a workgroup for windows of more
-// than kBigChunks chunks), the sparse kernel adds the first kSplitNnz sparse
-// nonzeros of those windows' rows and writes the sparse-only windows.  Last,
-// the pieces of rows longer than kSplitNnz: added with atomicAdd, or, in the
-// deterministic mode, summed into a workspace and added in piece order.
+// otherwise the sparse-row kernels run the sparse-only rows.  Other plans: the
+// streaming kernel (stile_stream.hip) stores the dense windows, with their
+// sparse parts when those are short, and the sparse-row kernels
+// (stile_sparse.hip) add the longer ones and write the sparse-only windows.
+// Last, the pieces of rows longer than kSplitNnz: added with atomicAdd, or, in
+// the deterministic mode, summed into a workspace and added by a reduce kernel.
+//
+// B is FP32, BF16 or FP16 (TB); every product and sum of the sparse part is
+// FP32 on B's exact values (FP64 sums for hub rows and pieces).
 // ---------------------------------------------------------------------------
-
-// Gathers in flight per lane group in the sparse and mixed slots.
-constexpr int kSparseDepth = 8;
-
-// Sum of v * B[col][n0+4j..+3] over nonzeros [r0, r1) of the sparse part.
-// DEPTH 8 keeps eight gathers in flight with the next ids prefetched; DEPTH 4
-// (four at a time) is for kernels whose register budget is tight.
-template <int DEPTH, typename TB>
-__device__ __forceinline__ float4 sparse_row_sum(const SpmmPlanDev& p, const TB* __restrict__ B,
-                                                 int64_t ldb, int N, int col, bool vec, int r0, int r1,
-                                                 bool compensated) {
-  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (!compensated) {
-    int q = r0;
-    // Eight gathers in flight, the next eight column ids fetched under them.
-    if (DEPTH >= 8 && q + 8 <= r1) {
-      int k[8];
-      float v[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        k[i] = p.res_cols[q + i];
-        v[i] = p.res_vals[q + i];
-      }
-      while (true) {
-        float4 b[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) b[i] = load_b4(B, ldb, k[i], col, N, vec);
-        const bool more = q + 16 <= r1;
-        int kn[8];
-        float vn[8];
-        if (more) {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            kn[i] = p.res_cols[q + 8 + i];
-            vn[i] = p.res_vals[q + 8 + i];
-          }
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          s.x += v[i] * b[i].x;
-          s.y += v[i] * b[i].y;
-          s.z += v[i] * b[i].z;
-          s.w += v[i] * b[i].w;
-        }
-        q += 8;
-        if (!more) break;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          k[i] = kn[i];
-          v[i] = vn[i];
-        }
-      }
-    }
-    for (; q + 4 <= r1; q += 4) {
-      const int k0 = p.res_cols[q], k1 = p.res_cols[q + 1], k2 = p.res_cols[q + 2], k3 = p.res_cols[q + 3];
-      const float v0 = p.res_vals[q], v1 = p.res_vals[q + 1], v2 = p.res_vals[q + 2], v3 = p.res_vals[q + 3];
-      const float4 b0 = load_b4(B, ldb, k0, col, N, vec);
-      const float4 b1 = load_b4(B, ldb, k1, col, N, vec);
-      const float4 b2 = load_b4(B, ldb, k2, col, N, vec);
-      const float4 b3 = load_b4(B, ldb, k3, col, N, vec);
-      s.x += v0 * b0.x; s.y += v0 * b0.y; s.z += v0 * b0.z; s.w += v0 * b0.w;
-      s.x += v1 * b1.x; s.y += v1 * b1.y; s.z += v1 * b1.z; s.w += v1 * b1.w;
-      s.x += v2 * b2.x; s.y += v2 * b2.y; s.z += v2 * b2.z; s.w += v2 * b2.w;
-      s.x += v3 * b3.x; s.y += v3 * b3.y; s.z += v3 * b3.z; s.w += v3 * b3.w;
-    }
-    for (; q < r1; ++q) {
-      const int k0 = p.res_cols[q];
-      const float v0 = p.res_vals[q];
-      const float4 b0 = load_b4(B, ldb, k0, col, N, vec);
-      s.x += v0 * b0.x; s.y += v0 * b0.y; s.z += v0 * b0.z; s.w += v0 * b0.w;
-    }
-  } else {
-    float4 cc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int q = r0; q < r1; ++q) {
-      const int k0 = p.res_cols[q];
-      const float v0 = p.res_vals[q];
-      const float4 b0 = load_b4(B, ldb, k0, col, N, vec);
-      neu_add(s.x, cc.x, v0 * b0.x);
-      neu_add(s.y, cc.y, v0 * b0.y);
-      neu_add(s.z, cc.z, v0 * b0.z);
-      neu_add(s.w, cc.w, v0 * b0.w);
-    }
-    s.x += cc.x; s.y += cc.y; s.z += cc.z; s.w += cc.w;
-  }
-  return s;
-}
 
 // Output rows of the 4 slots a lane group stores.  Loaded before any of the
 // window's C stores: vector-memory counters complete in issue order on
@@ -366,253 +263,6 @@ __device__ __forceinline__ void store_window(float* __restrict__ C, int64_t ldc,
   for (int i = 0; i < 4; ++i)
     if (sr.row[i] >= 0)
       store_c4<NT>(C, ldc, sr.row[i], col, N, vec, make_float4(acc[0][i], acc[1][i], acc[2][i], acc[3][i]));
-}
-
-// Slot of a dense window with a sparse part: C[row] += first kSplitNnz
-// nonzeros of the part (the streaming dense kernel stored C[row] before).
-template <typename TB>
-__device__ __forceinline__ void add_slot(const SpmmPlanDev& p, const TB* __restrict__ B, int64_t ldb, int N,
-                                         float* __restrict__ C, int64_t ldc, int col, bool vec, int slot) {
-  const int row = p.win_rows[slot];
-  const int r0 = p.res_ptr[slot], rend = p.res_ptr[slot + 1];
-  const int r1 = min(rend, r0 + kSplitNnz);
-  const float4 s = sparse_row_sum<kSparseDepth>(p, B, ldb, N, col, vec, r0, r1, rend - r0 > kHubNnz);
-  const float4 c = load_b4(C, ldc, row, col, N, vec);
-  store_c4(C, ldc, row, col, N, vec, make_float4(c.x + s.x, c.y + s.y, c.z + s.z, c.w + s.w));
-}
-
-template <int MODE>
-__device__ __forceinline__ void mfma_chunk(const SpmmPlanDev& p, int64_t c, int lane, const float4 (&b)[8],
-                                           f32x4 (&acc)[4]) {
-  if constexpr (MODE == 1) {
-    const bf16x8 a = reinterpret_cast<const bf16x8*>(p.tc_vals)[c * 64 + lane];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      bf16x8 bt;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) bt[e] = (__bf16)comp(b[e], t);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bt, acc[t], 0, 0, 0);
-    }
-  } else if constexpr (MODE == 2) {
-    const f16x8 a = reinterpret_cast<const f16x8*>(p.tc_vals)[c * 64 + lane];
-    const float sc = p.tc_scale[c];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      f16x8 bt;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) bt[e] = (_Float16)comp(b[e], t);
-      f32x4 tmp = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bt, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-      acc[t] += sc * tmp;
-    }
-  } else {
-    const float* ap = reinterpret_cast<const float*>(p.tc_vals) + (c * 64 + lane) * 8;
-    const float4 a0 = ld4(ap), a1 = ld4(ap + 4);
-    const float av[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], comp(b[e], t), acc[t], 0, 0, 0);
-    }
-  }
-}
-
-// B rows of one chunk for lane group g: 8 loads of four columns (addresses
-// from the chunk's column ids, already in registers).
-template <typename TB>
-__device__ __forceinline__ void load_chunk_b(const TB* __restrict__ B, int64_t ldb, int col, int N, bool vec,
-                                             const int4& ka, const int4& kb, float4 (&b)[8]) {
-  b[0] = load_b4(B, ldb, ka.x, col, N, vec);
-  b[1] = load_b4(B, ldb, ka.y, col, N, vec);
-  b[2] = load_b4(B, ldb, ka.z, col, N, vec);
-  b[3] = load_b4(B, ldb, ka.w, col, N, vec);
-  b[4] = load_b4(B, ldb, kb.x, col, N, vec);
-  b[5] = load_b4(B, ldb, kb.y, col, N, vec);
-  b[6] = load_b4(B, ldb, kb.z, col, N, vec);
-  b[7] = load_b4(B, ldb, kb.w, col, N, vec);
-}
-
-// Dense part of window w for this lane's columns.  Two chunks per step (16
-// independent B loads in flight) and the column ids of the next two chunks
-// fetched before the current step's B loads, so a step waits for one memory
-// latency instead of two.
-template <int MODE, typename TB>
-__device__ __forceinline__ void window_dense(const SpmmPlanDev& p, const TB* __restrict__ B, int64_t ldb,
-                                             int N, int col, bool vec, int c0, int c1, int lane,
-                                             f32x4 (&acc)[4]) {
-  const int g = lane >> 4;
-  if (c0 >= c1) return;
-  auto cols_of = [&](int c, int4& ka, int4& kb) {
-    const int4* cp = reinterpret_cast<const int4*>(p.tc_cols + (int64_t)c * 32 + g * 8);
-    ka = cp[0];
-    kb = cp[1];
-  };
-  int4 ka0, kb0, ka1, kb1;
-  cols_of(c0, ka0, kb0);
-  if (c0 + 1 < c1) cols_of(c0 + 1, ka1, kb1); else { ka1 = ka0; kb1 = kb0; }
-  int c = c0;
-  for (; c + 1 < c1; c += 2) {
-    int4 na0 = ka0, nb0 = kb0, na1 = ka1, nb1 = kb1;
-    if (c + 2 < c1) cols_of(c + 2, na0, nb0);
-    if (c + 3 < c1) cols_of(c + 3, na1, nb1);
-    float4 b0[8], b1[8];
-    load_chunk_b(B, ldb, col, N, vec, ka0, kb0, b0);
-    load_chunk_b(B, ldb, col, N, vec, ka1, kb1, b1);
-    mfma_chunk<MODE>(p, c, lane, b0, acc);
-    mfma_chunk<MODE>(p, c + 1, lane, b1, acc);
-    ka0 = na0; kb0 = nb0; ka1 = na1; kb1 = nb1;
-  }
-  if (c < c1) {
-    float4 b0[8];
-    load_chunk_b(B, ldb, col, N, vec, ka0, kb0, b0);
-    mfma_chunk<MODE>(p, c, lane, b0, acc);
-  }
-}
-
-template <int MODE, typename TB>
-__device__ __forceinline__ void hyb_spmm_window(const SpmmPlanDev& p, const TB* __restrict__ B, int64_t ldb,
-                                                int N, float* __restrict__ C, int64_t ldc, int w, int n0,
-                                                bool vec) {
-  const int lane = threadIdx.x & 63;
-  const int g = lane >> 4;
-  const int j = lane & 15;
-  const int col = n0 + 4 * j;
-
-  const SlotRows sr = load_rows(p, w * 16 + g * 4);
-  f32x4 acc[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  window_dense<MODE>(p, B, ldb, N, col, vec, p.tc_ptr[w], p.tc_ptr[w + 1], lane, acc);
-  store_window(C, ldc, N, col, vec, sr, acc);
-}
-
-// Blocks [0, n_parts * nC) each run one (part of a huge window, 64 columns):
-// they add their partial rows into C with atomicAdd (C rows zeroed before),
-// or, with ws (deterministic mode), store them to ws[part][16][N] for
-// hyb_spmm_part_reduce_kernel.  The next big_blocks each run one (big window,
-// 64 columns): wave v takes the v-th contiguous share of the window's chunks,
-// waves 1.. leave their partial sums in LDS and wave 0 adds them in wave
-// order and stores the 16 rows.  The other blocks run kBigWaves waves each
-// over the remaining dense windows [W_big, W_tc), one wave per window and 64
-// columns.
-template <int MODE, typename TB>
-__global__ __launch_bounds__(kBigWaves * 64) void hyb_spmm_kernel(SpmmPlanDev p, const TB* __restrict__ B,
-                                                                  int64_t ldb, int N, float* __restrict__ C,
-                                                                  int64_t ldc, int nC, int big_blocks,
-                                                                  bool vec, float* __restrict__ ws) {
-  __shared__ f32x4 part[kBigWaves - 1][4][64];
-  const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
-  const int huge_blocks = p.n_parts * nC;
-  const bool in_huge = (int)blockIdx.x < huge_blocks;
-  if (in_huge || (int)blockIdx.x < huge_blocks + big_blocks) {
-    int w, col, c0, c1, pt = 0;
-    if (in_huge) {
-      pt = blockIdx.x / nC;
-      w = p.part_win[pt];
-      col = (blockIdx.x - pt * nC) * 64 + 4 * (lane & 15);
-      c0 = p.part_c0[pt];
-      c1 = p.part_c1[pt];
-    } else {
-      w = p.W_huge + (int)(blockIdx.x - huge_blocks) / nC;
-      col = (int)(blockIdx.x - huge_blocks - (w - p.W_huge) * nC) * 64 + 4 * (lane & 15);
-      c0 = p.tc_ptr[w];
-      c1 = p.tc_ptr[w + 1];
-    }
-    const int share = (c1 - c0 + kBigWaves - 1) / kBigWaves;
-    const int a = min(c0 + wv * share, c1), b = min(a + share, c1);
-    SlotRows sr;
-    if (wv == 0) sr = load_rows(p, w * 16 + (lane >> 4) * 4);
-    f32x4 acc[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    with_vec(vec, [&](auto V) { window_dense<MODE>(p, B, ldb, N, col, V, a, b, lane, acc); });
-    if (wv > 0) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) part[wv - 1][t][lane] = acc[t];
-    }
-    __syncthreads();
-    if (wv != 0) return;
-    for (int v = 0; v < kBigWaves - 1; ++v) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) acc[t] += part[v][t][lane];
-    }
-    if (!in_huge) {
-      store_window(C, ldc, N, col, vec, sr, acc);
-      return;
-    }
-    if (ws) {
-      // partial rows of the part: ws[pt][slot 4g+i][col..col+3]
-      const int g = lane >> 4;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        store_c4(ws + (int64_t)pt * 16 * N, N, 4 * g + i, col, N, vec,
-                 make_float4(acc[0][i], acc[1][i], acc[2][i], acc[3][i]));
-      return;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (sr.row[i] < 0) continue;
-      float* cp = C + (int64_t)sr.row[i] * ldc + col;
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-        if (col + t < N) atomicAdd(cp + t, acc[t][i]);
-    }
-    return;
-  }
-  const int64_t wave = (int64_t)(blockIdx.x - huge_blocks - big_blocks) * kBigWaves + wv;
-  if (wave >= (int64_t)(p.W_tc - p.W_big) * nC) return;
-  const int w = p.W_big + (int)(wave / nC);
-  const int n0 = (int)(wave - (int64_t)(w - p.W_big) * nC) * 64;
-  with_vec(vec, [&](auto V) { hyb_spmm_window<MODE>(p, B, ldb, N, C, ldc, w, n0, V); });
-}
-
-// Deterministic mode: C rows of huge window w = sum of its parts' partial
-// rows in part order.  One wave per (huge window, 64 columns).
-__global__ __launch_bounds__(256) void hyb_spmm_part_reduce_kernel(SpmmPlanDev p, int N, float* __restrict__ C,
-                                                                   int64_t ldc, int nC, bool vec,
-                                                                   const float* __restrict__ ws) {
-  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  if (wave >= (int64_t)p.W_huge * nC) return;
-  const int w = (int)(wave / nC);
-  const int lane = threadIdx.x & 63, g = lane >> 4;
-  const int col = (int)(wave - (int64_t)w * nC) * 64 + 4 * (lane & 15);
-  const SlotRows sr = load_rows(p, w * 16 + g * 4);
-  const int q0 = p.hw_p0[w], q1 = p.hw_p0[w + 1];
-  float4 acc[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int q = q0; q < q1; ++q) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float4 v = load_b4(ws + (int64_t)q * 16 * N, N, 4 * g + i, col, N, vec);
-      acc[i].x += v.x; acc[i].y += v.y; acc[i].z += v.z; acc[i].w += v.w;
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    if (sr.row[i] >= 0) store_c4(C, ldc, sr.row[i], col, N, vec, acc[i]);
-}
-
-// Sparse parts of the dense windows' rows after the streaming kernel, one row
-// per lane group: the n_mix slots of dense windows, four per wave and 64
-// columns, added to the stored dense rows.  Waves go column chunk by column
-// chunk.
-// (256, 7): 71 VGPRs, no spills, 7 waves per SIMD instead of 6; the row
-// gathers are latency-bound.
-template <typename TB>
-__global__ __launch_bounds__(256, 7) void hyb_spmm_sparse_kernel(SpmmPlanDev p, const TB* __restrict__ B,
-                                                              int64_t ldb, int N, float* __restrict__ C,
-                                                              int64_t ldc, int nC, bool vec, int n_mix) {
-  const int lane = threadIdx.x & 63;
-  const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int64_t per = (n_mix + 3) / 4;
-  const int cch = (int)(wave / per);
-  if (cch >= nC) return;
-  const int q = (int)(wave - cch * per);
-  const int col = cch * 64 + 4 * (lane & 15);
-  const int m = q * 4 + (lane >> 4);
-  if (m < n_mix) with_vec(vec, [&](auto V) { add_slot(p, B, ldb, N, C, ldc, col, V, p.mix_slot[m]); });
 }
 
 // Sparse-only rows for launches with too few rows to fill the GPU at one row
@@ -1285,48 +935,16 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   } else if (p.W_tc > 0) {
-    if (p.n_parts > 0 && !det) {
-      hipError_t e = launch_zero_window_rows(p, p.W_huge, C, ldc, N, s);
-      if (e != hipSuccess) return e;
-    }
-    const int64_t big_blocks = (int64_t)(p.W_big - p.W_huge) * nC;
-    const int64_t blocks = (int64_t)p.n_parts * nC + big_blocks +
-                           ((int64_t)(p.W_tc - p.W_big) * nC + kBigWaves - 1) / kBigWaves;
-    if (blocks > INT32_MAX) return hipErrorInvalidValue;
-    dim3 grid((unsigned)blocks), block(kBigWaves * 64);
-    const int bb = (int)big_blocks;
-    switch (p.blk_dtype) {
-      case 1:
-        hipLaunchKernelGGL((hyb_spmm_kernel<1, TB>), grid, block, 0, s, p, B, ldb, N, C, ldc, nC, bb, vec,
-                           ws_parts);
-        break;
-      case 2:
-        hipLaunchKernelGGL((hyb_spmm_kernel<2, TB>), grid, block, 0, s, p, B, ldb, N, C, ldc, nC, bb, vec,
-                           ws_parts);
-        break;
-      default:
-        hipLaunchKernelGGL((hyb_spmm_kernel<0, TB>), grid, block, 0, s, p, B, ldb, N, C, ldc, nC, bb, vec,
-                           ws_parts);
-        break;
-    }
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_stream(p, B, ldb, N, C, ldc, vec, ws_parts, s);
     if (e != hipSuccess) return e;
-    if (det && p.W_huge > 0) {
-      const int64_t waves = (int64_t)p.W_huge * nC;
-      hipLaunchKernelGGL(hyb_spmm_part_reduce_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, p, N, C,
-                         ldc, nC, vec, ws_parts);
-      e = hipGetLastError();
-      if (e != hipSuccess) return e;
-    }
   }
-  // Sparse-only rows (unless folded) by wave tasks, or, when there are fewer
-  // than 16,384 (row, 64 columns) of 8 or more nonzeros on average, one of those
-  // per wave with all its gathers in flight at once; then, unless the LDS kernel
-  // added them, the sparse parts of the dense windows' rows.
-  const int n_mix = lds ? 0 : p.n_mix;
+  // Sparse-only rows (unless they were the LDS launch's tail) by wave tasks, or,
+  // when there are fewer than 16,384 (row, 64 columns) of 8 or more nonzeros on
+  // average, one of those per wave with all its gathers in flight at once.  The
+  // sparse parts of dense windows come first in the task list, when neither the
+  // LDS nor the streaming kernel added them.
   const int64_t so_left = fold ? 0 : so_rows;
   const bool split = so_left > 0 && so_left * nC / 4 < 4096 && p.nnz_sparse_only >= 8 * so_left;
-  const int64_t sparse_waves = (int64_t)((n_mix + 3) / 4) * nC;
   if (split) {
     const int64_t blocks = (so_rows * nC + 3) / 4;
     hipLaunchKernelGGL(hyb_spmm_sparse_split_kernel<TB>, dim3((unsigned)blocks), dim3(256), 0, s, p, B, ldb, N, C,
@@ -1334,16 +952,9 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  if (so_left > 0 && !split) {
-    hipError_t e = launch_sparse_rows(p, B, ldb, N, C, ldc, vec, s);
-    if (e != hipSuccess) return e;
-  }
-  if (sparse_waves > 0) {
-    const int64_t blocks = (sparse_waves + 3) / 4;
-    if (blocks > INT32_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(hyb_spmm_sparse_kernel<TB>, dim3((unsigned)blocks), dim3(256), 0, s, p, B, ldb, N, C, ldc,
-                       nC, vec, n_mix);
-    hipError_t e = hipGetLastError();
+  {
+    hipError_t e = launch_sparse_rows(p, B, ldb, N, C, ldc, vec, lds ? p.n_mix_tasks : 0,
+                                      so_left > 0 && !split ? p.n_row_tasks : p.n_mix_tasks, s);
     if (e != hipSuccess) return e;
   }
   // Pieces of long rows.  The LDS kernel summed its windows' rows whole, so

@@ -649,35 +649,38 @@ void attention_order(const std::vector<int32_t>& win_rows, const std::vector<int
 }
 
 // Wave tasks over the slots [s0, s1) (SpmmPlanDev::row_tasks): consecutive
-// slots until they hold `target` entries, a row of more than kSplitNnz alone.
+// slots until they hold `target` entries, a row of more than kSplitNnz alone,
+// appended to out.
 // 64 entries a task hide the latencies at its start and end; a plan with fewer
 // than 8,192 such tasks (eight waves per SIMD) takes smaller ones, down to 16
 // entries.  Tasks of 128 entries and more run first, so that none of them
 // starts when the others are done.
-std::vector<int32_t> sparse_row_tasks(const std::vector<int64_t>& ptr, int64_t s0, int64_t s1) {
+void sparse_row_tasks(const std::vector<int64_t>& ptr, int64_t s0, int64_t s1, int32_t flags,
+                      std::vector<int32_t>& out) {
   const int64_t target = std::min<int64_t>(64, std::max<int64_t>(16, (ptr[s1] - ptr[s0]) / 8192));
   constexpr int64_t kMaxSlots = 64, kLong = 128;
   std::vector<std::array<int32_t, 2>> tasks;
   int64_t a = s0;
+  auto close = [&](int64_t s, int32_t f) {
+    // slots without entries are only stored (0), not added
+    if (s > a && !((flags & stile::kTaskAdd) && ptr[s] == ptr[a]))
+      tasks.push_back({(int32_t)a, (int32_t)s | flags | f});
+    a = s;
+  };
   for (int64_t s = s0; s < s1; ++s) {
     const int64_t len = ptr[s + 1] - ptr[s];
     if (len > stile::kSplitNnz) {
-      if (s > a) tasks.push_back({(int32_t)a, (int32_t)s});
-      tasks.push_back({(int32_t)s, (int32_t)((uint32_t)(s + 1) | (len > stile::kHubNnz ? 0x80000000u : 0u))});
-      a = s + 1;
+      close(s, 0);
+      close(s + 1, len > stile::kHubNnz ? stile::kTaskHub : 0);
     } else if (ptr[s + 1] - ptr[a] >= target || s + 1 - a >= kMaxSlots) {
-      tasks.push_back({(int32_t)a, (int32_t)(s + 1)});
-      a = s + 1;
+      close(s + 1, 0);
     }
   }
-  if (a < s1) tasks.push_back({(int32_t)a, (int32_t)s1});
+  close(s1, 0);
   std::stable_partition(tasks.begin(), tasks.end(), [&](const std::array<int32_t, 2>& t) {
-    return ptr[t[1] & 0x7fffffff] - ptr[t[0]] >= kLong;
+    return ptr[t[1] & stile::kTaskSlots] - ptr[t[0]] >= kLong;
   });
-  std::vector<int32_t> out;
-  out.reserve(tasks.size() * 2);
   for (const auto& t : tasks) out.insert(out.end(), t.begin(), t.end());
-  return out;
 }
 
 int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan** out) {
@@ -735,8 +738,9 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
     }
   }
   auto has_chunks = [&](int32_t w) { return !bd.win_cols[w].empty() || !bd.win_scat[w].empty(); };
-  // Windows with more than stile::kBigChunks dense chunks first (most chunks first,
-  // W_big of them), then the other windows with dense chunks (W_tc in all),
+  // Windows with more than stile::kLongChunks dense chunks first (most chunks
+  // first; W_big of them have more than kBigChunks), then the other windows with
+  // dense chunks (W_tc in all),
   // then the sparse-only windows; the kernels map the kinds onto waves
   // differently.
   std::vector<int32_t> order(W);
@@ -757,10 +761,10 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
     for (int32_t w = 0; w < W; ++w) mat[w] = window_matrix(bd, w);
     std::stable_sort(order.begin(), order.begin() + W_tc, [&](int32_t a, int32_t b) { return mat[a] < mat[b]; });
   } else {
-    auto big_end = std::stable_partition(order.begin(), order.begin() + W_tc,
-                                         [&](int32_t w) { return nch(w) > stile::kBigChunks; });
-    std::stable_sort(order.begin(), big_end, [&](int32_t a, int32_t b) { return nch(a) > nch(b); });
-    W_big = (int32_t)(big_end - order.begin());
+    auto long_end = std::stable_partition(order.begin(), order.begin() + W_tc,
+                                          [&](int32_t w) { return nch(w) > stile::kLongChunks; });
+    std::stable_sort(order.begin(), long_end, [&](int32_t a, int32_t b) { return nch(a) > nch(b); });
+    while (W_big < W_tc && nch(order[W_big]) > stile::kBigChunks) ++W_big;
     while (W_huge < W_big && nch(order[W_huge]) > stile::kHugeChunks) ++W_huge;
   }
   {
@@ -814,11 +818,17 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
       if (bd.has_ids) res_ids[q] = bd.s_id[src[q]];
     }
   }
-  // Slots of dense windows that also have a sparse part: the sparse kernel
-  // adds those parts to the rows the dense kernels stored.
-  std::vector<int32_t> mix_slot;
+  // Slots of dense windows that also have a sparse part: summed with the window
+  // when they are short (fold_mix), else added to the rows the streaming kernel
+  // stored by the sparse rows' tasks.
+  int32_t n_mix = 0;
+  int64_t longest_mix = 0;
   for (int64_t sl = 0; sl < (int64_t)W_tc * 16; ++sl)
-    if (cnt[sl + 1] > cnt[sl]) mix_slot.push_back((int32_t)sl);
+    if (cnt[sl + 1] > cnt[sl]) {
+      ++n_mix;
+      longest_mix = std::max(longest_mix, cnt[sl + 1] - cnt[sl]);
+    }
+  const bool fold_mix = longest_mix <= stile::kFoldMaxLen;
   // Long rows: the window pass takes the first kSplitNnz nonzeros of a slot,
   // the rest is cut into pieces of kSplitNnz for the fix-up kernel.
   // Pieces are in slot order, so those of dense windows' slots come first
@@ -845,7 +855,10 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
     }
   }
 
-  const std::vector<int32_t> row_tasks = sparse_row_tasks(cnt, (int64_t)W_tc * 16, (int64_t)W * 16);
+  std::vector<int32_t> row_tasks;
+  if (!fold_mix) sparse_row_tasks(cnt, 0, (int64_t)W_tc * 16, stile::kTaskAdd, row_tasks);
+  const int32_t n_mix_tasks = (int32_t)(row_tasks.size() / 2);
+  sparse_row_tasks(cnt, (int64_t)W_tc * 16, (int64_t)W * 16, 0, row_tasks);
 
   if (lds_ok)
     for (int32_t w = 0; w < W_tc; ++w) order_chunk_slots(bd.win_cols[w], bd.inst_cols[window_matrix(bd, w)]);
@@ -1041,7 +1054,6 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   const size_t o_pend = lay.add(piece_end.size() * 4);
   const size_t o_tcids = lay.add(tc_ids.size() * 4);
   const size_t o_resids = lay.add(res_ids.size() * 4);
-  const size_t o_mix = lay.add(mix_slot.size() * 4);
   const size_t o_mask = lay.add(tc_mask.size() * 4);
   const size_t o_pwin = lay.add(part_win.size() * 4);
   const size_t o_pc0 = lay.add(part_c0.size() * 4);
@@ -1086,7 +1098,6 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   blob.put(o_pend, piece_end.data(), piece_end.size() * 4);
   blob.put(o_tcids, tc_ids.data(), tc_ids.size() * 4);
   blob.put(o_resids, res_ids.data(), res_ids.size() * 4);
-  blob.put(o_mix, mix_slot.data(), mix_slot.size() * 4);
   blob.put(o_mask, tc_mask.data(), tc_mask.size() * 4);
   blob.put(o_pwin, part_win.data(), part_win.size() * 4);
   blob.put(o_pc0, part_c0.data(), part_c0.size() * 4);
@@ -1121,14 +1132,16 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   d.W_tc = W_tc;
   d.W_big = W_big;
   d.W_huge = W_huge;
+  d.chunks_small = tc_ptr[W_tc] - tc_ptr[W_big];
   d.n_parts = (int32_t)part_win.size();
   d.part_win = dptr<int32_t>(plan, o_pwin);
   d.part_c0 = dptr<int32_t>(plan, o_pc0);
   d.part_c1 = dptr<int32_t>(plan, o_pc1);
   d.n_row_tasks = (int32_t)(row_tasks.size() / 2);
+  d.n_mix_tasks = n_mix_tasks;
   d.row_tasks = dptr<int2>(plan, o_rtask);
-  d.n_mix = (int32_t)mix_slot.size();
-  d.mix_slot = dptr<int32_t>(plan, o_mix);
+  d.n_mix = n_mix;
+  d.fold_mix = fold_mix ? 1 : 0;
   d.tc_mask = tc_mask.empty() ? nullptr : dptr<uint32_t>(plan, o_mask);
   d.lds_units = lds_units.empty() ? nullptr : dptr<int4>(plan, o_units);
   for (int t = 0; t < stile::kLdsLists; ++t) {
