@@ -174,7 +174,7 @@ def load():
 
 
 def _check(rc):
-    if rc != 0:
+    if rc:
         msg = load().stile_last_error().decode(errors="replace")
         raise StileError(f"libstile_hip error {rc}: {msg}")
 
@@ -183,9 +183,38 @@ def _ptr(arr, ctype):
     return arr.ctypes.data_as(ctypes.POINTER(ctype))
 
 
-def _stream(t=None):
+# torch, imported on the first call that needs it, its current-stream handle by
+# device index and the STILE_BLK_* code of each type of B
+_torch = _raw_stream = None
+_b_codes = {}
+
+
+def _load_torch():
+    global _torch, _raw_stream
     import torch
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device if t is not None else None).cuda_stream)
+    _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
+                          lambda index: torch.cuda.current_stream(index).cuda_stream)
+    _b_codes.update({torch.float32: STILE_BLK_F32, torch.bfloat16: STILE_BLK_BF16, torch.float16: STILE_BLK_F16})
+    _torch = torch
+    return torch
+
+
+def _stream(t):
+    """The HIP stream handle of torch's current stream on t's device.  (The
+    public torch.cuda.current_stream builds a Stream object per call, 2 of the 9
+    us a small product spent on the host.)"""
+    if _torch is None:
+        _load_torch()
+    return _raw_stream(t.device.index)
+
+
+def _b_code(dtype):
+    if _torch is None:
+        _load_torch()
+    code = _b_codes.get(dtype)
+    if code is None:
+        raise StileError("B must be float32, bfloat16 or float16")
+    return code
 
 
 def blk_dtype_code(dtype):
@@ -213,7 +242,7 @@ def _dev_check(*ts):
     for t in ts:
         if not t.is_cuda:
             raise StileError("libstile_hip kernels take device tensors")
-    if len({t.device for t in ts}) > 1:
+    if len(ts) > 1 and any(t.device != ts[0].device for t in ts):
         raise StileError("all tensors of a call must be on one device")
 
 
@@ -228,14 +257,14 @@ def _out(out, shape, device, what="out"):
     """The output tensor of a call: a new one, or the caller's after checking
     what the kernel will write through its pointer (float32, on `device`,
     exactly `shape`, rows contiguous)."""
-    import torch
+    torch = _torch or _load_torch()
     if out is None:
         return torch.empty(shape, device=device, dtype=torch.float32)
     if not out.is_cuda or out.device != device:
         raise StileError(f"{what} must be on {device}")
     if out.dtype != torch.float32:
         raise StileError(f"{what} must be float32")
-    if tuple(out.shape) != tuple(shape):
+    if out.shape != shape:
         raise StileError(f"{what} has shape {tuple(out.shape)}, expected {tuple(shape)}")
     if out.numel() > 0 and out.stride(-1) != 1:
         raise StileError(f"{what} must have unit stride along its last dimension")
@@ -429,7 +458,7 @@ class Plan:
     def run_attention(self, Q, K, V, scale, out=None):
         """out = softmax(scale * Q K^T on the masks) V; Q, K, V BF16 (rows x 64,
         rows = the stacked instances), out FP32."""
-        import torch
+        torch = _torch or _load_torch()
         if not getattr(self, "attention_plan", False):
             raise StileError("not an attention plan")
         _dev_check(Q, K, V)
@@ -458,7 +487,7 @@ class Plan:
 
     def set_values(self, vals):
         """Refresh A's values (device float32, A's CSR order) without rebuilding."""
-        import torch
+        torch = _torch or _load_torch()
         if self.kind != "spmm":
             raise StileError("not an SpMM plan")
         _dev_check(vals)
@@ -484,18 +513,17 @@ class Plan:
         C float32.  deterministic: split rows and huge windows are summed in a
         fixed order through `workspace` (a device uint8/any tensor of at least
         workspace_bytes(N, True) bytes; allocated here when not given)."""
-        import torch
         if self.kind != "spmm":
             raise StileError("not an SpMM plan")
-        _dev_check(B)
-        codes = {torch.float32: STILE_BLK_F32, torch.bfloat16: STILE_BLK_BF16, torch.float16: STILE_BLK_F16}
-        if B.dtype not in codes:
-            raise StileError("B must be float32, bfloat16 or float16")
-        if B.shape[0] != self.K:
-            raise StileError(f"B has {B.shape[0]} rows, the plan's A has {self.K} columns")
+        if not B.is_cuda:
+            raise StileError("libstile_hip kernels take device tensors")
+        code = _b_code(B.dtype)
+        shape = B.shape
+        if shape[0] != self.K:
+            raise StileError(f"B has {shape[0]} rows, the plan's A has {self.K} columns")
         if B.stride(1) != 1:
             B = B.contiguous()
-        N = B.shape[1]
+        N = shape[1]
         C = _out(out, (self.M, N), B.device)
         flags, ws_ptr, ws_bytes = 0, None, 0
         if deterministic:
@@ -503,13 +531,14 @@ class Plan:
             need = self.workspace_bytes(N, True)
             if need > 0:
                 if workspace is None:
+                    import torch
                     workspace = torch.empty(need, dtype=torch.uint8, device=B.device)
                 _dev_check(workspace)
                 if workspace.device != B.device or not workspace.is_contiguous():
                     raise StileError("workspace must be a contiguous tensor on B's device")
                 ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
-        _check(load().stile_spmm_run_ex(self._h, codes[B.dtype], B.data_ptr(), B.stride(0), N, C.data_ptr(),
-                                        C.stride(0), flags, ws_ptr, ws_bytes, _stream(B)))
+        _check((_lib or load()).stile_spmm_run_ex(self._h, code, B.data_ptr(), B.stride(0), N, C.data_ptr(),
+                                                  C.stride(0), flags, ws_ptr, ws_bytes, _stream(B)))
         return C
 
     def run_spmm_noalloc(self, B, out, deterministic=False):
@@ -520,21 +549,19 @@ class Plan:
         if self.kind != "spmm":
             raise StileError("not an SpMM plan")
         _dev_check(B, out)
-        codes = {torch.float32: STILE_BLK_F32, torch.bfloat16: STILE_BLK_BF16, torch.float16: STILE_BLK_F16}
-        if B.dtype not in codes:
-            raise StileError("B must be float32, bfloat16 or float16")
+        code = _b_code(B.dtype)
         if B.shape[0] != self.K or B.stride(1) != 1:
             raise StileError(f"B must be {self.K} x N with contiguous rows")
         N = B.shape[1]
         if out.dtype != torch.float32 or tuple(out.shape) != (self.M, N) or out.stride(1) != 1:
             raise StileError(f"out must be a float32 {self.M} x {N} tensor with contiguous rows")
-        _check(load().stile_spmm_run_noalloc(self._h, codes[B.dtype], B.data_ptr(), B.stride(0), N, out.data_ptr(),
+        _check(load().stile_spmm_run_noalloc(self._h, code, B.data_ptr(), B.stride(0), N, out.data_ptr(),
                                              out.stride(0), STILE_RUN_DETERMINISTIC if deterministic else 0,
                                              _stream(B)))
         return out
 
     def run_sddmm(self, X, Y, out=None):
-        import torch
+        torch = _torch or _load_torch()
         if self.kind != "sddmm":
             raise StileError("not an SDDMM plan")
         _dev_check(X, Y)
