@@ -208,6 +208,15 @@ int stile_ell_buckets_spmm_f32(const StileEllBucket* buckets, int32_t count, int
 int stile_csr_row_softmax_f32(int32_t M, const int32_t* indptr, const float* in, float* out, float scale,
                               void* stream);
 
+/* out (F x Fg, FP32) = H^T G for tall H (M x F) and G (M x Fg): the weight
+ * gradient of a dense layer over M rows (the GCN layer's H.W; the reference has
+ * no backward pass).  Rows are summed in slabs through `workspace`
+ * (stile_tall_tn_workspace_bytes, 16-byte aligned), the slabs in a fixed order.
+ * STILE_E_UNSUPPORTED when H or G spans 4 GiB or more. */
+int stile_tall_tn_workspace_bytes(int32_t M, int32_t F, int32_t Fg, int64_t* bytes);
+int stile_tall_tn_f32(int32_t M, int32_t F, int32_t Fg, const float* H, int64_t ldh, const float* G, int64_t ldg,
+                      float* out, int64_t ldo, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Build a hybrid SpMM plan from the packed groups (host pointers; copied).
  * The plan regroups every group's products by 16-row output window, so C
  * needs no zero-fill and most rows are stored once with a fixed summation

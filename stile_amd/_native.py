@@ -90,6 +90,11 @@ _SIGNATURES = {
                                            ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p]),
     "stile_csr_row_softmax_f32": (ctypes.c_int, [ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p,
                                                  ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p]),
+    "stile_tall_tn_workspace_bytes": (ctypes.c_int, [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
+                                                     ctypes.POINTER(ctypes.c_int64)]),
+    "stile_tall_tn_f32": (ctypes.c_int, [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p,
+                                         ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+                                         ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]),
     "stile_plan_create_spmm": (ctypes.c_int, [ctypes.POINTER(StileSpmmPack), ctypes.c_int32,
                                               ctypes.POINTER(ctypes.c_void_p)]),
     "stile_plan_create_spmm_batched": (ctypes.c_int, [ctypes.POINTER(StileSpmmPack), ctypes.c_int32,
@@ -339,6 +344,24 @@ def csr_row_softmax_f32(indptr, vals, scale=1.0, out=None):
     o = _out(out, tuple(vals.shape), vals.device)
     _check(load().stile_csr_row_softmax_f32(indptr.numel() - 1, indptr.data_ptr(), vals.data_ptr(),
                                             o.data_ptr(), float(scale), _stream(vals)))
+    return o
+
+
+def tall_tn_f32(H, G):
+    """H^T G for tall float32 H (M x F) and G (M x Fg) on the device."""
+    torch = _torch or _load_torch()
+    _dev_check(H, G)
+    if H.dtype != torch.float32 or G.dtype != torch.float32 or H.shape[0] != G.shape[0]:
+        raise StileError("tall_tn_f32 takes float32 H and G of as many rows")
+    (M, F), Fg = H.shape, G.shape[1]
+    H = H if H.stride(1) == 1 and H.stride(0) >= F else H.contiguous()
+    G = G if G.stride(1) == 1 and G.stride(0) >= Fg else G.contiguous()
+    n = ctypes.c_int64()
+    _check(load().stile_tall_tn_workspace_bytes(M, F, Fg, ctypes.byref(n)))
+    ws = torch.empty(n.value, dtype=torch.uint8, device=H.device)
+    o = torch.empty((F, Fg), dtype=torch.float32, device=H.device)
+    _check(load().stile_tall_tn_f32(M, F, Fg, H.data_ptr(), H.stride(0), G.data_ptr(), G.stride(0), o.data_ptr(),
+                                    o.stride(0), ws.data_ptr(), n.value, _stream(H)))
     return o
 
 

@@ -181,12 +181,35 @@ def sddmm(op, X, Y):
     return op.sddmm(X, Y)
 
 
+# Rows from which the tall kernel takes H^T G: below them the vendor's GEMM has
+# little to reduce (see _tall_kernel_fits).
+_TALL_ROWS = 4096
+
+
+def _tall_kernel_fits(H, G):
+    """True where the library's own H^T G runs instead of a GEMM: plain float32
+    device tensors, outside tracing and outside a backward pass that is itself
+    differentiated, with many more rows than output entries per side (a GEMM has
+    one workgroup per output tile and a few splits of the rows; measured at
+    M = 32768, F = Fg = 256: 138 us against 56)."""
+    if not (type(H) is type(G) is torch.Tensor and H.is_cuda and G.is_cuda and H.dtype == G.dtype == torch.float32):
+        return False
+    M, F, Fg = H.shape[0], H.shape[1], G.shape[1]
+    span = (1 << 32) - (1 << 20)
+    return (M >= _TALL_ROWS and 0 < F <= M // 32 and 0 < Fg <= M // 32 and F * Fg <= 1 << 20
+            and 4 * M * max(H.stride(0), F) < span and 4 * M * max(G.stride(0), Fg) < span
+            and not torch.is_grad_enabled() and not torch.compiler.is_compiling())
+
+
 def _split_k_tn(H, G, slab_rows=16384):
-    """H^T G for tall H, G (M x F, M >> F).  As one GEMM the reduction over M
-    leaves the library a handful of F x F output tiles for the whole GPU; cut
-    into M / slab_rows slabs it is one batched product with that many times
-    more tiles, then a sum over the slabs.  FP32 only (other dtypes, and M not
-    a multiple of the slab, take the single GEMM)."""
+    """H^T G for tall H, G (M x F, M >> F).  On the device a kernel of the
+    library (_tall_kernel_fits); else, as one GEMM the reduction over M leaves
+    the library a handful of F x F output tiles: cut into M / slab_rows slabs it
+    is one batched product with that many times more tiles, then a sum over the
+    slabs.  FP32 only (other dtypes, and M not a multiple of the slab, take the
+    single GEMM)."""
+    if _tall_kernel_fits(H, G):
+        return _native.tall_tn_f32(H, G)
     M = H.shape[0]
     if H.dtype != torch.float32 or G.dtype != torch.float32 or M % slab_rows or M < 4 * slab_rows:
         return H.t() @ G

@@ -256,6 +256,12 @@ template <typename TB>
 hipError_t launch_stream(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc, bool vec,
                          float* ws, hipStream_t s);
 
+// out (F x Fg) = H^T G over M rows; ws: slabs * F * Fg floats (tall_slabs gives
+// the slab count and rows per slab).  H and G each span less than 4 GiB.
+int tall_slabs(int M, int F, int Fg, int* slab);
+hipError_t launch_tall_tn(int M, int F, int Fg, const float* H, int64_t ldh, const float* G, int64_t ldg, float* out,
+                          int64_t ldo, float* ws, hipStream_t s);
+
 // Zero-fill kernels (used instead of hipMemsetAsync so that every *_run call
 // records only kernel nodes under HIP graph capture).
 hipError_t launch_fill_zero(float* p, int64_t n, hipStream_t s);

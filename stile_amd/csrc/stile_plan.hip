@@ -1495,6 +1495,39 @@ int stile_ell_buckets_spmm_f32(const StileEllBucket* buckets, int32_t count, int
   return STILE_OK;
 }
 
+int stile_tall_tn_workspace_bytes(int32_t M, int32_t F, int32_t Fg, int64_t* bytes) {
+  if (!bytes) return fail(STILE_E_INVALID, "null output pointer");
+  if (M < 0 || F < 0 || Fg < 0) return fail(STILE_E_INVALID, "negative size");
+  int slab = 0;
+  *bytes = M == 0 || F == 0 || Fg == 0 ? 0 : (int64_t)stile::tall_slabs(M, F, Fg, &slab) * F * Fg * 4;
+  return STILE_OK;
+}
+
+int stile_tall_tn_f32(int32_t M, int32_t F, int32_t Fg, const float* H, int64_t ldh, const float* G, int64_t ldg,
+                      float* out, int64_t ldo, void* workspace, int64_t workspace_bytes, void* stream) {
+  int64_t need = 0;
+  const int rc = stile_tall_tn_workspace_bytes(M, F, Fg, &need);
+  if (rc != STILE_OK) return rc;
+  if (F == 0 || Fg == 0) return STILE_OK;
+  if (!out) return fail(STILE_E_INVALID, "null pointer");
+  if (ldo < Fg) return fail(STILE_E_INVALID, "leading dimension smaller than the row");
+  if (M == 0) {
+    hipError_t e = stile::launch_fill_zero_2d(out, F, Fg, ldo, (hipStream_t)stream);
+    return e == hipSuccess ? STILE_OK : hip_fail(e, "fill_zero launch");
+  }
+  if (!H || !G) return fail(STILE_E_INVALID, "null pointer");
+  if (ldh < F || ldg < Fg) return fail(STILE_E_INVALID, "leading dimension smaller than the row");
+  const int64_t limit = (int64_t)1 << 32;
+  if (ldh >= (1 << 30) || ldg >= (1 << 30) || ((int64_t)(M - 1) * ldh + F) * 4 >= limit ||
+      ((int64_t)(M - 1) * ldg + Fg) * 4 >= limit)
+    return fail(STILE_E_UNSUPPORTED, "H and G must span less than 4 GiB");
+  if (!workspace || workspace_bytes < need)
+    return fail(STILE_E_INVALID, "workspace smaller than stile_tall_tn_workspace_bytes");
+  hipError_t e = stile::launch_tall_tn(M, F, Fg, H, ldh, G, ldg, out, ldo, static_cast<float*>(workspace),
+                                       (hipStream_t)stream);
+  return e == hipSuccess ? STILE_OK : hip_fail(e, "tall_tn launch");
+}
+
 int stile_plan_create_spmm(const StileSpmmPack* pack, int32_t blk_dtype, StilePlan** out) {
   return create_spmm(pack, 1, blk_dtype, out);
 }
