@@ -173,17 +173,16 @@ __global__ __launch_bounds__(256) void hyb_spmm_piece_reduce_kernel(SpmmPlanDev 
 
 namespace {
 
-// Columns per lane: the widest of 4, 2 and 1 that wastes no more lanes than
-// the others (64 * VW columns per wave) and leaves at least kFewWaves waves
-// for `waves` of them per column chunk (two per SIMD: below that a wave's
-// latency is what the launch takes, and narrower waves are more of them).
+// Columns per lane: 2 for more than 64 columns when that leaves at least
+// kFewWaves waves (two per SIMD: below that a wave's latency is what the launch
+// takes, and narrower waves are more of them), else 1.  (4 columns per lane: 105
+// registers and half the waves in flight; R-MAT scale 16, N = 256: 172 against
+// 161 us.  Sixteen entries a batch: 265 us, the scalar registers spill.  One
+// slice of columns per XCD: no change.)
 constexpr int64_t kFewWaves = 2048;
 int row_width(int N, int64_t waves) {
-  auto chunks = [&](int vw) { return (N + 64 * vw - 1) / (64 * vw); };
-  int best = 1;
-  for (int vw = 2; vw <= 4; vw *= 2)
-    if (chunks(vw) * vw <= chunks(best) * best && waves * chunks(vw) >= kFewWaves) best = vw;
-  return best;
+  const int64_t chunks = (N + 127) / 128;
+  return N > 64 && waves * chunks >= kFewWaves ? 2 : 1;
 }
 
 // f(VW, kVec, kBuf) with all three as compile-time constants.
@@ -201,9 +200,7 @@ void with_width(int vw, bool vec, bool buf, F&& f) {
     else
       h(std::false_type{});
   };
-  if (vw == 4)
-    g(std::integral_constant<int, 4>{});
-  else if (vw == 2)
+  if (vw == 2)
     g(std::integral_constant<int, 2>{});
   else
     g(std::integral_constant<int, 1>{});
