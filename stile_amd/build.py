@@ -14,7 +14,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "libstile_hip.so")
 SOURCES = ["stile_kernels.hip", "stile_attention.hip", "stile_sparse.hip",
-           "stile_stream.hip", "stile_dense.hip", "stile_plan.hip"]
+           "stile_stream.hip", "stile_dense.hip", "stile_sddmm.hip",
+           "stile_plan.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"

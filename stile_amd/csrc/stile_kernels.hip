@@ -985,154 +985,6 @@ hipError_t launch_hyb_spmm(const SpmmPlanDev& p, int b_dtype, const void* B, int
 }
 
 // ---------------------------------------------------------------------------
-// Hybrid fused SDDMM.  Waves [0, waves1d) run the 1D entries (segments of LPE
-// lanes, kSddmmU consecutive entries each); the remaining waves each run one
-// dense 16x16 block:
-// lane l = 16g + j loads float4 slices of X[rows[j]] and Y[cols[j]] at
-// features kb + 4g .. kb + 4g + 3 and feeds component e to MFMA e
-// (v_mfma_f32_16x16x4_f32, so k-slot g of MFMA e is feature kb + 4g + e).
-// The 16x16 result goes through LDS to the sampled scatter.
-// ---------------------------------------------------------------------------
-constexpr int kSddmmU = 4;
-
-template <int LPE>
-// (256, 8): registers for 8 waves per SIMD (59 VGPRs, no spills); the 1D
-// entries are latency-bound gathers and more waves in flight measured faster
-// (R-MAT scale 16, K = 32: 16.3 -> 15.2 us with every entry in the 1D part).
-__global__ __launch_bounds__(256, 8) void hyb_sddmm_kernel(SddmmPlanDev p,
-                                                        const float* __restrict__ X,
-                                                        int64_t ldx,
-                                                        const float* __restrict__ Y,
-                                                        int64_t ldy, int Kf,
-                                                        float* __restrict__ out,
-                                                        int waves1d, bool vec) {
-  __shared__ float blk[4][256];
-  const int lane = threadIdx.x & 63;
-  const int wib = threadIdx.x >> 6;
-  const int wave = blockIdx.x * 4 + wib;
-  if (wave < waves1d) {
-    // a segment of LPE lanes computes kSddmmU consecutive entries, their
-    // index loads and row gathers all in flight together
-    constexpr int EPW = 64 / LPE;
-    const int sub = lane % LPE;
-    const int e0 = (wave * EPW + lane / LPE) * kSddmmU;
-    if (e0 >= p.n1d) return;
-    int row[kSddmmU], col[kSddmmU], dst[kSddmmU];
-#pragma unroll
-    for (int u = 0; u < kSddmmU; ++u) {
-      const int e = min(e0 + u, p.n1d - 1);
-      row[u] = p.e_row[e];
-      col[u] = p.e_col[e];
-      dst[u] = p.e_out[e];
-    }
-    float s[kSddmmU];
-#pragma unroll
-    for (int u = 0; u < kSddmmU; ++u) s[u] = 0.f;
-    if (vec) {
-      // consecutive entries of one row (CSR order) share the X load; an
-      // entry whose row repeats skips its load and takes the previous X
-      // value in a select after every load is issued (a copy inside the
-      // branch would wait for the previous load before the next one)
-      bool same[kSddmmU];
-#pragma unroll
-      for (int u = 0; u < kSddmmU; ++u) same[u] = u > 0 && row[u] == row[u - 1];
-      for (int k = 4 * sub; k < Kf; k += 4 * LPE) {
-        float4 a[kSddmmU], b[kSddmmU];
-#pragma unroll
-        for (int u = 0; u < kSddmmU; ++u) {
-          if (!same[u]) a[u] = ld4(X + (int64_t)row[u] * ldx + k);
-          b[u] = ld4(Y + (int64_t)col[u] * ldy + k);
-        }
-#pragma unroll
-        for (int u = 1; u < kSddmmU; ++u)
-          if (same[u]) a[u] = a[u - 1];
-#pragma unroll
-        for (int u = 0; u < kSddmmU; ++u) s[u] += a[u].x * b[u].x + a[u].y * b[u].y + a[u].z * b[u].z + a[u].w * b[u].w;
-      }
-    } else {
-      for (int k = sub; k < Kf; k += LPE) {
-#pragma unroll
-        for (int u = 0; u < kSddmmU; ++u) s[u] += X[(int64_t)row[u] * ldx + k] * Y[(int64_t)col[u] * ldy + k];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kSddmmU; ++u) {
-#pragma unroll
-      for (int off = LPE / 2; off > 0; off >>= 1) s[u] += __shfl_xor(s[u], off, LPE);
-    }
-    if (sub == 0) {
-#pragma unroll
-      for (int u = 0; u < kSddmmU; ++u)
-        if (e0 + u < p.n1d) out[dst[u]] = s[u];
-    }
-    return;
-  }
-  const int b = wave - waves1d;
-  if (b >= p.nblk) return;
-  const int g = lane >> 4, j = lane & 15;
-  const float* xr = X + (int64_t)p.blk_rows[b * 16 + j] * ldx;
-  const float* yr = Y + (int64_t)p.blk_cols[b * 16 + j] * ldy;
-  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int kb = 0; kb < Kf; kb += 16) {
-    const int k = kb + 4 * g;
-    float4 xa, ya;
-    if (vec && k + 3 < Kf) {
-      xa = ld4(xr + k);
-      ya = ld4(yr + k);
-    } else {
-      xa.x = k < Kf ? xr[k] : 0.f;         ya.x = k < Kf ? yr[k] : 0.f;
-      xa.y = k + 1 < Kf ? xr[k + 1] : 0.f; ya.y = k + 1 < Kf ? yr[k + 1] : 0.f;
-      xa.z = k + 2 < Kf ? xr[k + 2] : 0.f; ya.z = k + 2 < Kf ? yr[k + 2] : 0.f;
-      xa.w = k + 3 < Kf ? xr[k + 3] : 0.f; ya.w = k + 3 < Kf ? yr[k + 3] : 0.f;
-    }
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.x, ya.x, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.y, ya.y, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.z, ya.z, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa.w, ya.w, acc, 0, 0, 0);
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) blk[wib][(4 * g + i) * 16 + j] = acc[i];
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const int s0 = p.blk_ptr[b], s1 = p.blk_ptr[b + 1];
-  for (int s = s0 + lane; s < s1; s += 64) out[p.blk_out[s]] = blk[wib][p.blk_pos[s]];
-}
-
-hipError_t launch_hyb_sddmm(const SddmmPlanDev& p, const float* X,
-                            int64_t ldx, const float* Y, int64_t ldy, int Kf,
-                            float* out, hipStream_t s) {
-  const bool vec = (Kf % 4 == 0) && (ldx % 4 == 0) && (ldy % 4 == 0) &&
-                   ((reinterpret_cast<uintptr_t>(X) & 15) == 0) &&
-                   ((reinterpret_cast<uintptr_t>(Y) & 15) == 0);
-  int lpe = vec ? Kf / 4 : Kf;
-  if (lpe > 16) lpe = 16;
-  if (lpe < 1) lpe = 1;
-  int l = 1;
-  while (l * 2 <= lpe) l *= 2;
-  lpe = l;
-  const int epw = 64 / lpe * kSddmmU;
-  const int waves1d = (p.n1d + epw - 1) / epw;
-  const int64_t waves = (int64_t)waves1d + p.nblk;
-  if (waves == 0) return hipSuccess;
-  dim3 grid((unsigned)((waves + 3) / 4));
-#define STILE_HSDDMM_CASE(L)                                                  \
-  case L:                                                                     \
-    hipLaunchKernelGGL(hyb_sddmm_kernel<L>, grid, dim3(256), 0, s, p, X, ldx, \
-                       Y, ldy, Kf, out, waves1d, vec);                        \
-    break;
-  switch (lpe) {
-    STILE_HSDDMM_CASE(1)
-    STILE_HSDDMM_CASE(2)
-    STILE_HSDDMM_CASE(4)
-    STILE_HSDDMM_CASE(8)
-    STILE_HSDDMM_CASE(16)
-  }
-#undef STILE_HSDDMM_CASE
-  return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
 // Row softmax over CSR rows: one wave per row; max and sum reduced with xor
 // shuffles across the 64 lanes.
 // ---------------------------------------------------------------------------

@@ -1333,6 +1333,13 @@ int create_sddmm(const StileSddmmPack* packs, int32_t count, int32_t blk_dtype, 
   bd.M = (int32_t)roff;
   bd.N = (int32_t)coff;
   bd.nnz = (int32_t)ooff;
+  // the kernel reads the entries' ids four at a time
+  const size_t n1d = bd.e_row.size();
+  while (bd.e_row.size() % 4) {
+    bd.e_row.push_back(bd.e_row.back());
+    bd.e_col.push_back(bd.e_col.back());
+    bd.e_out.push_back(bd.e_out.back());
+  }
   Layout lay;
   const size_t o_er = lay.add(bd.e_row.size() * 4), o_ec = lay.add(bd.e_col.size() * 4),
                o_eo = lay.add(bd.e_out.size() * 4), o_br = lay.add(bd.b_rows.size() * 4),
@@ -1362,7 +1369,7 @@ int create_sddmm(const StileSddmmPack* packs, int32_t count, int32_t blk_dtype, 
   d.M = bd.M;
   d.N = bd.N;
   d.nnz = bd.nnz;
-  d.n1d = (int32_t)bd.e_row.size();
+  d.n1d = (int32_t)n1d;
   d.nblk = (int32_t)(bd.b_ptr.size() - 1);
   d.blk_dtype = blk_dtype;
   d.e_row = dptr<int32_t>(plan, o_er);
@@ -1381,7 +1388,7 @@ int create_sddmm(const StileSddmmPack* packs, int32_t count, int32_t blk_dtype, 
   in.num_windows = 0;
   in.num_chunks = d.nblk;
   in.block_nnz = (int64_t)bd.b_pos.size();
-  in.sparse_nnz = (int64_t)bd.e_row.size();
+  in.sparse_nnz = (int64_t)n1d;
   in.device_bytes = (int64_t)plan->dev_bytes;
   in.hub_rows = 0;
   in.num_split = 0;
