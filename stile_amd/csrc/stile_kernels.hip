@@ -380,11 +380,48 @@ constexpr int kLdsThreads = 1024;
 //     (one v_perm_b32 and one 4-byte write each);
 //   FP32 B: piece (row r, columns 4m .. 4m + 3) -> column 4m + t to position
 //     16t + m (two packed conversions, four 2-byte writes).
+// kStore == 2 (rows of B or C not aligned for a vector of columns): the same
+// pieces at any alignment, 16-byte loads that need element alignment only; a
+// piece that reaches past N is read from N - 8, or N - 4, on and shifted.  Only
+// widths below one piece are read element by element, which is 8 times the
+// loads (and as many store instructions, see store_window_lds): 3072 x 768
+// times N = 4093, BF16 B: 36.3 us element by element, 18.3 so (N = 4096, every
+// row aligned: 13.2); 1024 x 1000, N = 333: 12.8 and 7.4, FP32 B 20.6 and 11.7;
+// 24-layer batch of 1024 x 4096 layers, N = 101: 95.5 and 70.6.
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+// Eight 16-bit columns from c0 on of a row of N >= 8, zero at or beyond N.
 template <typename TB>
+__device__ __forceinline__ uint4 load8_any(const TB* __restrict__ row, int c0, int N) {
+  const int c = min(c0, N - 8);
+  const u32x4_any d = *reinterpret_cast<const u32x4_any*>(row + c);
+  uint64_t lo = ((uint64_t)d[1] << 32) | d[0], hi = ((uint64_t)d[3] << 32) | d[2];
+  const int s = 16 * (c0 - c);  // bits to drop: 0 inside the row
+  if (s > 0) {
+    lo = s >= 64 ? hi >> (s & 63) : (lo >> s) | (hi << (64 - s));
+    hi = s >= 64 ? 0 : hi >> s;
+    if (s >= 128) lo = 0;
+  }
+  return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+}
+
+// Four FP32 columns from c0 on of a row of N >= 4, zero at or beyond N.
+__device__ __forceinline__ float4 load4_any(const float* __restrict__ row, int c0, int N) {
+  const int c = min(c0, N - 4), s = c0 - c;
+  const f32x4_any d = *reinterpret_cast<const f32x4_any*>(row + c);
+  float4 r = make_float4(d[0], d[1], d[2], d[3]);
+  if (s & 1) r = make_float4(r.y, r.z, r.w, 0.f);
+  if (s & 2) r = make_float4(r.z, r.w, 0.f, 0.f);
+  return s >= 4 ? make_float4(0.f, 0.f, 0.f, 0.f) : r;
+}
+
+template <typename TB, int kStore>
 __device__ __forceinline__ void stage_b(lds_u8* lds, const TB* __restrict__ B, int64_t ldb, int koff, int ksz,
                                         int n0, int N, bool vec, bool vec16) {
+  constexpr bool kAny = kStore == 2;
   if constexpr (!std::is_same<TB, float>::value) {
-    if (vec16) {
+    if (vec16 || (kAny && N >= 8)) {
       constexpr int U = kLdsMaxK * 8 / kLdsThreads;
       const int items = ksz * 8;
       uint4 d[U];
@@ -392,8 +429,11 @@ __device__ __forceinline__ void stage_b(lds_u8* lds, const TB* __restrict__ B, i
       for (int u = 0; u < U; ++u) {
         const int it = min((int)threadIdx.x + u * kLdsThreads, items - 1);
         const int c0 = n0 + 8 * (it & 7);
-        d[u] = c0 < N ? *reinterpret_cast<const uint4*>(B + (int64_t)(koff + (it >> 3)) * ldb + c0)
-                      : make_uint4(0, 0, 0, 0);
+        const TB* row = B + (int64_t)(koff + (it >> 3)) * ldb;
+        if constexpr (kAny)
+          d[u] = load8_any(row, c0, N);
+        else
+          d[u] = c0 < N ? *reinterpret_cast<const uint4*>(row + c0) : make_uint4(0, 0, 0, 0);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -427,7 +467,11 @@ __device__ __forceinline__ void stage_b(lds_u8* lds, const TB* __restrict__ B, i
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int it = min(base + u * kLdsThreads, items - 1);
-      f[u] = load_b4(B, ldb, koff + (it >> 4), n0 + 4 * (it & 15), N, vec);
+      if constexpr (kAny && std::is_same<TB, float>::value)
+        f[u] = N >= 4 ? load4_any(B + (int64_t)(koff + (it >> 4)) * ldb, n0 + 4 * (it & 15), N)
+                      : load_b4(B, ldb, koff + (it >> 4), n0 + 4 * (it & 15), N, false);
+      else
+        f[u] = load_b4(B, ldb, koff + (it >> 4), n0 + 4 * (it & 15), N, vec);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -549,32 +593,49 @@ __device__ __forceinline__ void sparse_round(const TB* __restrict__ B, int64_t l
 typedef float f32v4_t __attribute__((ext_vector_type(4)));
 
 // The window's rows as float4 stores of four columns each, one per row.
-// kVec (C rows 16-byte aligned, N a multiple of 4, C below 2 GiB): buffer
+// kStore 1 (C rows 16-byte aligned, N a multiple of 4, C below 2 GiB): buffer
 // stores with L2 write-through (sc1) over a descriptor of [C, C + cbytes),
 // measured 4 % faster on the block-pruned layer at N = 4096 than
 // non-temporal global stores; stores that fall outside C (rows of -1,
 // columns at or beyond N) get an offset past the descriptor, which the
 // hardware drops, so every lane issues the same stores on every path.
 // Otherwise store_window.
-template <bool kVec>
+// kStore 2 (any alignment and width): the quads that lie inside a row as
+// unaligned 16-byte stores, the columns of the one that reaches past N one by
+// one, in the items that hold it.
+template <int kStore>
 __device__ __forceinline__ void store_window_lds(float* __restrict__ C, int64_t ldc, int N, int col, bool vec,
                                                  int cbytes, const SlotRows& sr, const f32x4 (&acc)[4]) {
-  if constexpr (kVec) {
+  if constexpr (kStore > 0) {
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(C, 0, cbytes, 0x00020000);
     constexpr uint32_t kOut = 0x80000000u;  // past every descriptor (cbytes < 2^31)
+    auto at = [&](int i) { return ((uint32_t)sr.row[i] * (uint32_t)ldc + (uint32_t)col) * 4u; };
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const bool ok = sr.row[i] >= 0 && col < N;
-      const uint32_t off = ok ? ((uint32_t)sr.row[i] * (uint32_t)ldc + (uint32_t)col) * 4u : kOut;
-      __builtin_amdgcn_raw_buffer_store_b128(f32v4_t{acc[0][i], acc[1][i], acc[2][i], acc[3][i]}, rs, (int)off, 0,
-                                            16);
+      const bool ok = sr.row[i] >= 0 && (kStore == 1 ? col < N : col + 3 < N);
+      __builtin_amdgcn_raw_buffer_store_b128(f32v4_t{acc[0][i], acc[1][i], acc[2][i], acc[3][i]}, rs,
+                                             (int)(ok ? at(i) : kOut), 0, 16);
+    }
+    if constexpr (kStore == 2) {
+      // wave-uniform: the item's 64 columns end past N inside a quad
+      const int n0 = col - 4 * (int)(threadIdx.x & 15);
+      if ((N & 3) && n0 + 64 > N) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int t = 0; t < 3; ++t) {
+            const bool ok = sr.row[i] >= 0 && col + 3 >= N && col + t < N;
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[t][i]), rs, (int)(ok ? at(i) + 4u * t : kOut), 0,
+                                                  16);
+          }
+      }
     }
   } else {
     store_window<true>(C, ldc, N, col, vec, sr, acc);
   }
 }
 
-template <typename TB, bool kMixed, bool kVec, bool kSc>
+template <typename TB, bool kMixed, int kStore, bool kSc>
 __device__ __forceinline__ void lds_item(const SpmmPlanDev& p, const int32_t* __restrict__ tc_ptr,
                                          const int32_t* __restrict__ sp_off, const uint32_t* __restrict__ tc_kind,
                                          const int32_t* __restrict__ win_r0, const int4* __restrict__ units,
@@ -663,7 +724,7 @@ __device__ __forceinline__ void lds_item(const SpmmPlanDev& p, const int32_t* __
       request_rounds(so0);
     }
   }
-  stage_b(lds, B, ldb, koff, ksz, n0, N, vec, vec16);
+  stage_b<TB, kStore>(lds, B, ldb, koff, ksz, n0, N, vec, vec16);
   if (has) r2 = load_tr_chunk(p, min(c_beg + 2, last), cidx, lane, is_sc(min(c_beg + 2, last)));
   __syncthreads();
   if (!has) return;
@@ -702,7 +763,7 @@ __device__ __forceinline__ void lds_item(const SpmmPlanDev& p, const int32_t* __
       cur = load_win(p, w * 16 + g * 4);
       asm volatile("" : "+v"(cur.row[0]), "+v"(cur.row[1]), "+v"(cur.row[2]), "+v"(cur.row[3]));
     }
-    store_window_lds<kVec>(C, ldc, N, col, vec, cbytes, cur, acc);
+    store_window_lds<kStore>(C, ldc, N, col, vec, cbytes, cur, acc);
   };
   TrChunk r3;
   int c = c_beg;
@@ -755,7 +816,7 @@ __device__ __forceinline__ void lds_item(const SpmmPlanDev& p, const int32_t* __
 // 16i + 15 of tail_tasks.  Under the XCD grouping those are the last slot of
 // each XCD, which holds the fewest items when a range does not divide evenly;
 // one-item launches add tail blocks past the items when CUs are free.
-template <bool kLoop, typename TB, bool kMixed, bool kVec>
+template <bool kLoop, typename TB, bool kMixed, int kStore>
 __global__ __launch_bounds__(kLdsThreads) void hyb_spmm_lds_bf16_kernel(SpmmPlanDev p,
                                                                         const int32_t* __restrict__ tc_ptr,
                                                                         const int32_t* __restrict__ sp_off,
@@ -772,10 +833,10 @@ __global__ __launch_bounds__(kLdsThreads) void hyb_spmm_lds_bf16_kernel(SpmmPlan
   const int tb = (int)gridDim.x - 1 - (int)blockIdx.x;
   auto run = [&](int item) {  // tc_kind: kernel-uniform
     if (tc_kind)
-      lds_item<TB, kMixed, kVec, true>(p, tc_ptr, sp_off, tc_kind, win_r0, units, B, ldb, N, C, ldc, nC, vec, vec16,
+      lds_item<TB, kMixed, kStore, true>(p, tc_ptr, sp_off, tc_kind, win_r0, units, B, ldb, N, C, ldc, nC, vec, vec16,
                                        cbytes, item, lds);
     else
-      lds_item<TB, kMixed, kVec, false>(p, tc_ptr, sp_off, tc_kind, win_r0, units, B, ldb, N, C, ldc, nC, vec,
+      lds_item<TB, kMixed, kStore, false>(p, tc_ptr, sp_off, tc_kind, win_r0, units, B, ldb, N, C, ldc, nC, vec,
                                         vec16, cbytes, item, lds);
   };
   if (!kLoop) {
@@ -812,10 +873,12 @@ __global__ __launch_bounds__(kLdsThreads) void hyb_spmm_lds_bf16_kernel(SpmmPlan
 
 template <bool kLoop, typename TB>
 static void set_lds_bytes(int bytes) {
-  for (const void* f : {reinterpret_cast<const void*>(hyb_spmm_lds_bf16_kernel<kLoop, TB, false, false>),
-                        reinterpret_cast<const void*>(hyb_spmm_lds_bf16_kernel<kLoop, TB, true, false>),
-                        reinterpret_cast<const void*>(hyb_spmm_lds_bf16_kernel<kLoop, TB, false, true>),
-                        reinterpret_cast<const void*>(hyb_spmm_lds_bf16_kernel<kLoop, TB, true, true>)})
+  for (const void* f : {reinterpret_cast<const void*>(hyb_spmm_lds_bf16_kernel<kLoop, TB, false, 0>),
+                        reinterpret_cast<const void*>(hyb_spmm_lds_bf16_kernel<kLoop, TB, true, 0>),
+                        reinterpret_cast<const void*>(hyb_spmm_lds_bf16_kernel<kLoop, TB, false, 1>),
+                        reinterpret_cast<const void*>(hyb_spmm_lds_bf16_kernel<kLoop, TB, true, 1>),
+                        reinterpret_cast<const void*>(hyb_spmm_lds_bf16_kernel<kLoop, TB, false, 2>),
+                        reinterpret_cast<const void*>(hyb_spmm_lds_bf16_kernel<kLoop, TB, true, 2>)})
     (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
@@ -909,8 +972,8 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
     const size_t lds_bytes = (size_t)p.lds_max_k * kLdsRowBytes;
     const int4* units = p.lds_units + p.lds_off[t];
     const bool mixed = p.n_mix > 0 && p.sp_off != nullptr;
-    // C addressed by a buffer descriptor (the kVec variants) when its extent
-    // is below 2 GiB
+    // C addressed by a buffer descriptor (kStore 1, 2) when its extent is below
+    // 2 GiB
     const int64_t c_extent = ((int64_t)(p.M - 1) * ldc + N) * 4;
     const int cbytes = p.M > 0 && c_extent < ((int64_t)1 << 31) ? (int)c_extent : 0;
 #define STILE_LDS_LAUNCH1(LOOP, MIX, VEC)                                                                    \
@@ -921,9 +984,11 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
 #define STILE_LDS_LAUNCH(LOOP, MIX)                \
   do {                                             \
     if (vec && cbytes > 0)                         \
-      STILE_LDS_LAUNCH1(LOOP, MIX, true);          \
+      STILE_LDS_LAUNCH1(LOOP, MIX, 1);             \
+    else if (cbytes > 0)                           \
+      STILE_LDS_LAUNCH1(LOOP, MIX, 2);             \
     else                                           \
-      STILE_LDS_LAUNCH1(LOOP, MIX, false);         \
+      STILE_LDS_LAUNCH1(LOOP, MIX, 0);             \
   } while (0)
     if (items <= cus) {
       if (mixed) STILE_LDS_LAUNCH(false, true); else STILE_LDS_LAUNCH(false, false);
