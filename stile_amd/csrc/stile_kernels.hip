@@ -609,12 +609,12 @@ __device__ __forceinline__ void store_window_lds(float* __restrict__ C, int64_t 
   if constexpr (kStore > 0) {
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(C, 0, cbytes, 0x00020000);
     constexpr uint32_t kOut = 0x80000000u;  // past every descriptor (cbytes < 2^31)
-    auto at = [&](int i) { return ((uint32_t)sr.row[i] * (uint32_t)ldc + (uint32_t)col) * 4u; };
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const bool ok = sr.row[i] >= 0 && (kStore == 1 ? col < N : col + 3 < N);
-      __builtin_amdgcn_raw_buffer_store_b128(f32v4_t{acc[0][i], acc[1][i], acc[2][i], acc[3][i]}, rs,
-                                             (int)(ok ? at(i) : kOut), 0, 16);
+      const bool ok = sr.row[i] >= 0 && (kStore == 1 ? col : col + 3) < N;
+      const uint32_t off = ok ? ((uint32_t)sr.row[i] * (uint32_t)ldc + (uint32_t)col) * 4u : kOut;
+      __builtin_amdgcn_raw_buffer_store_b128(f32v4_t{acc[0][i], acc[1][i], acc[2][i], acc[3][i]}, rs, (int)off, 0,
+                                            16);
     }
     if constexpr (kStore == 2) {
       // wave-uniform: the item's 64 columns end past N inside a quad
@@ -625,8 +625,8 @@ __device__ __forceinline__ void store_window_lds(float* __restrict__ C, int64_t 
 #pragma unroll
           for (int t = 0; t < 3; ++t) {
             const bool ok = sr.row[i] >= 0 && col + 3 >= N && col + t < N;
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[t][i]), rs, (int)(ok ? at(i) + 4u * t : kOut), 0,
-                                                  16);
+            const uint32_t off = ok ? ((uint32_t)sr.row[i] * (uint32_t)ldc + (uint32_t)(col + t)) * 4u : kOut;
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[t][i]), rs, (int)off, 0, 16);
           }
       }
     }
