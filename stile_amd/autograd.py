@@ -207,11 +207,19 @@ def _split_k_tn(H, G, slab_rows=16384):
     the library a handful of F x F output tiles: cut into M / slab_rows slabs it
     is one batched product with that many times more tiles, then a sum over the
     slabs.  FP32 only (other dtypes, and M not a multiple of the slab, take the
-    single GEMM)."""
-    if _tall_kernel_fits(H, G):
-        return _native.tall_tn_f32(H, G)
+    single GEMM).
+
+    The slabs also run where they fill the GPU and their tiles, fitted to F, beat
+    the kernel's 128 x 64 ones, in us for F = Fg, kernel / slabs: M = 2^20, F = 32
+    179 / 56, 64 182 / 146, 128 334 / 299, 256 1140 / 953; M = 2^18 71 / 51, 71 /
+    47, 101 / 104, 326 / 264; M = 2^17 55 / 55, 55 / 92, 65 / 66, 165 / 139; M =
+    2^16 49 / 56, 48 / 90, 48 / 98, 92 / 115."""
     M = H.shape[0]
-    if H.dtype != torch.float32 or G.dtype != torch.float32 or M % slab_rows or M < 4 * slab_rows:
+    slabs = H.dtype == G.dtype == torch.float32 and M % slab_rows == 0 and M >= 4 * slab_rows
+    beaten = slabs and (M >= 1 << 18 or M * H.shape[1] * G.shape[1] >= 1 << 33)
+    if not beaten and _tall_kernel_fits(H, G):
+        return _native.tall_tn_f32(H, G)
+    if not slabs:
         return H.t() @ G
     S = M // slab_rows
     H3 = H.contiguous().view(S, slab_rows, H.shape[1])

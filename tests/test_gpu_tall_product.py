@@ -53,3 +53,15 @@ def test_gradient_of_the_gradient(cuda):
     dW, = torch.autograd.grad(tall_matmul(H, W), (W,), dY, create_graph=True)
     dH, = torch.autograd.grad(dW.sum(), (H,))
     assert torch.allclose(dH, dY.detach().sum(1, keepdim=True).expand_as(dH), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("M", [65536, 131072, 131073, 262143, 262144])
+@pytest.mark.parametrize("F,Fg", [(24, 32), (256, 256)])
+def test_backward_where_row_slabs_take_over(cuda, M, F, Fg):
+    g = torch.Generator(device=cuda)
+    g.manual_seed(M + F)
+    H = torch.randn(M, F, device=cuda, generator=g, requires_grad=True)
+    W = torch.randn(F, Fg, device=cuda, generator=g, requires_grad=True)
+    dY = torch.randn(M, Fg, device=cuda, generator=g)
+    print("tall backward", M, F, Fg, flush=True)
+    _check(H.detach(), dY, torch.autograd.grad(tall_matmul(H, W), W, dY)[0])
