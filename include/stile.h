@@ -151,10 +151,10 @@ typedef struct {
   int64_t sparse_nnz;     /* nonzeros carried by the FP32 1D/ELL path */
   int64_t device_bytes;   /* bytes of plan buffers resident on the device */
   int32_t hub_rows;       /* rows with > 4096 sparse nonzeros: each 256-term
-                             piece of such a row is summed with Neumaier
-                             compensation, the pieces then plainly added */
+                             piece of such a row is summed in FP64, the
+                             pieces then added in FP32 */
   int32_t num_split;      /* SpMM: pieces of rows with > 256 sparse nonzeros,
-                             added to C by the fix-up kernel */
+                             added to C by the pieces kernel */
 } StilePlanInfo;
 
 /* ---------------------------------------------------------------------------

@@ -8,13 +8,14 @@
 namespace stile {
 
 // Hub rows: a row whose sparse (non-MFMA) part has more than this many
-// nonzeros is summed with compensated (Neumaier) FP32 arithmetic, per
-// kSplitNnz-term piece (the pieces are then added plainly).
+// nonzeros is summed in FP64 per kSplitNnz-term piece (the pieces are then
+// added plainly in FP32); the plain CSR kernels and the one-wave-per-row
+// kernel of few rows sum it with compensated (Neumaier) FP32 arithmetic.
 constexpr int kHubNnz = 4096;
 
 // Rows whose sparse part is longer than this are cut: the window pass sums
-// the first kSplitNnz nonzeros, the rest go to pieces of kSplitNnz that a
-// fix-up kernel adds with atomicAdd after the window pass (in deterministic
+// the first kSplitNnz nonzeros, the rest go to pieces of kSplitNnz that the
+// pieces kernel adds with atomicAdd after the window pass (in deterministic
 // mode: stores to a workspace, summed in piece order by a reduce kernel).
 constexpr int kSplitNnz = 256;
 
@@ -103,7 +104,7 @@ struct SpmmPlanDev {
   const int32_t* piece_row;  // [npieces] output row
   const int32_t* piece_beg;  // [npieces] range in res_cols/res_vals
   const int32_t* piece_end;
-  // execution order of the pieces for the fix-up kernel: within [0,
+  // execution order of the pieces for the pieces kernel: within [0,
   // npieces_dense) and [npieces_dense, npieces), pieces by their first
   // column, so the pieces running together (of different long rows) gather
   // the same B rows ([npieces])

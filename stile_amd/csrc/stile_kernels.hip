@@ -1,19 +1,20 @@
 // HIP kernels of libstile_hip.so for MI355X (gfx950, CDNA4, wave64).
 //
-// Four kernel templates:
+// The kernels here:
 //   csr_spmm_f32     plain CSR SpMM (the comparator; reference csrmm template,
 //                    MY_sparse/my_fuse_formats.py:1106-1152)
 //   csr_sddmm_f32    plain per-nonzero SDDMM (reference golden u_dot_v,
 //                    my_fuse_formats.py:4331-4341)
-//   hyb_spmm         hybrid fused SpMM: MFMA on dense 16-row blocks + FP32
-//                    sparse part, one wave per (16-row window, 64 columns),
-//                    every C row written once (replaces the fused ELL +
-//                    TensorCore templates, my_fuse_formats.py:1162-1291,
+//   hyb_spmm_lds     hybrid fused SpMM of BF16 plans with K <= kLdsMaxK: dense
+//                    16-row blocks on MFMA against B staged in LDS + the FP32
+//                    sparse part, every C row written once (replaces the fused
+//                    ELL + TensorCore templates, my_fuse_formats.py:1162-1291,
 //                    1444-1799, 2426-2465)
-//   hyb_sddmm        hybrid fused SDDMM: 1D entries as FP32 wave-segment dot
-//                    products + dense 16x16 blocks on MFMA with sampled
-//                    scatter (my_fuse_formats.py:2263-2317, 2324-2415,
-//                    2519-2560)
+//   sparse_split     few sparse rows: one wave per row and 64 columns
+//   row softmax, value refresh, ELL buckets (comparator), zero fills
+// and launch_hyb_spmm, which picks a product's kernels: these, the streaming
+// kernel (stile_stream.hip) and the sparse rows (stile_sparse.hip).  The SDDMM,
+// the fused attention and the tall product have files of their own.
 #include "stile_device.h"
 
 #include <algorithm>
@@ -274,7 +275,7 @@ __device__ __forceinline__ void store_window(float* __restrict__ C, int64_t ldc,
 // together.  Positions past r1 read the row's last entry with weight 0.
 // Fixed order: within a group u = 0..15 per round, then the xor-shuffle sum
 // over the four groups.  Rows with more than kHubNnz sparse nonzeros sum with
-// Neumaier compensation, as in finish_slot.
+// Neumaier compensation.
 template <typename TB>
 __device__ __forceinline__ void sparse_split_wave(const SpmmPlanDev& p, const TB* __restrict__ B, int64_t ldb,
                                                   int N, float* __restrict__ C, int64_t ldc, int nC, bool vec,

@@ -830,7 +830,7 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
     }
   const bool fold_mix = longest_mix <= stile::kFoldMaxLen;
   // Long rows: the window pass takes the first kSplitNnz nonzeros of a slot,
-  // the rest is cut into pieces of kSplitNnz for the fix-up kernel.
+  // the rest is cut into pieces of kSplitNnz for the pieces kernel.
   // Pieces are in slot order, so those of dense windows' slots come first
   // (npieces_dense); each split row's pieces are consecutive (srow_*).
   int32_t hub_rows = 0;
@@ -1039,7 +1039,7 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   const size_t o_resptr = lay.add(res_ptr.size() * 4);
   const size_t o_rescols = lay.add((res_cols.size() + stile::kRowPad) * 4);
   const size_t o_resvals = lay.add((res_vals.size() + stile::kRowPad) * 4);
-  // the fix-up kernel's piece order (see SpmmPlanDev::piece_exec)
+  // the pieces kernel's order (see SpmmPlanDev::piece_exec)
   std::vector<int32_t> piece_exec(piece_row.size());
   for (size_t q = 0; q < piece_exec.size(); ++q) piece_exec[q] = (int32_t)q;
   auto by_first_col = [&](int32_t a, int32_t b) {

@@ -21,7 +21,7 @@ namespace stile {
 // 2.55 M entries of this kernel take 115 us (11.3 TB/s of gathered rows); with
 // one row per 16-lane group, four rows of unequal length per wave and each
 // row's entries in sequence they took 444 us.  Scale 15, N = 250 (rows that are
-// not 16-byte aligned): 932 -> 88 us for the whole product.
+// not 16-byte aligned): 932 -> 83 us for the whole product.
 // ---------------------------------------------------------------------------
 constexpr int kRowBatch = 8;
 

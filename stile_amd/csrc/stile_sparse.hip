@@ -91,11 +91,13 @@ __global__ __launch_bounds__(256, 4) void hyb_spmm_rows_kernel(
 // to C with atomicAdd (C already holds the row's first kSplitNnz entries), or,
 // with ws (deterministic mode), stored to ws[piece][N] for the reduce kernel.
 // One workgroup per piece and 64 * VW columns, a quarter of the entries per
-// wave (a graph with few long rows has few pieces: 143 of them as one wave each
-// took 36 us on N = 256, as four 15 us), the waves' sums added in wave order.
+// wave, the waves' sums added in wave order: a graph with few long rows has few
+// pieces, and as one wave each they made the GCN layer's products (R-MAT scale
+// 16, N = 256) 12 us longer; in quarters the launch takes 6.6-7.1 us, 15.1
+// with the compensated FP32 sums it had before.
 // FP64 sums: one conversion and one v_fma_f64 (as fast as v_fma_f32 here) per
 // product against nine operations of a compensated FP32 sum, which bounded
-// this kernel (1.31 M entries, N = 128: 58 us).
+// this kernel (1.31 M entries, N = 128: 58 -> 49 us).
 template <typename TB, int VW, bool kVec, bool kBuf>
 __global__ __launch_bounds__(256, 4) void hyb_spmm_pieces_kernel(
     const int32_t* __restrict__ piece_exec, const int32_t* __restrict__ piece_row,
