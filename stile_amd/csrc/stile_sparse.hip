@@ -181,10 +181,22 @@ namespace {
 // registers and half the waves in flight; R-MAT scale 16, N = 256: 172 against
 // 161 us.  Sixteen entries a batch: 265 us, the scalar registers spill.  One
 // slice of columns per XCD: no change.)
+//
+// FP32 B whose 128 columns are more than twice the L2s together (8 x 4 MB): 1 as
+// well.  The launch runs column chunk by column chunk, and what one chunk's
+// gathers touch, half as much of B, is then found in L2 and MALL more often.  A
+// graph's whole product, FP32, N = 128, two columns per lane / one: scale 18 (128
+// columns are 128 MB) 430 / 366 us; 19: 938 / 793; 20: 2005 / 1709, N = 256 4000
+// / 3500.  Scale 17 (64 MB) gains or loses with the plan (with dense chunks 195 /
+// 183, sparse only 173 / 175, N = 200 306 / 332), smaller ones lose (16, N = 256:
+// 166 / 172).  16-bit B, whose two columns are those 256 bytes a gather, keeps
+// two at every size: scale 17 125 / 170, 20 1070 / 1297.
 constexpr int64_t kFewWaves = 2048;
-int row_width(int N, int64_t waves) {
+constexpr int64_t kWideBytes = 64 << 20;
+int row_width(int N, int K, int elem, int64_t waves) {
   const int64_t chunks = (N + 127) / 128;
-  return N > 64 && waves * chunks >= kFewWaves ? 2 : 1;
+  const bool wide = elem == 2 || (int64_t)K * 128 * elem <= kWideBytes;
+  return wide && N > 64 && waves * chunks >= kFewWaves ? 2 : 1;
 }
 
 // f(VW, kVec, kBuf) with all three as compile-time constants.
@@ -215,7 +227,7 @@ hipError_t launch_sparse_rows(const SpmmPlanDev& p, const TB* B, int64_t ldb, in
                               int t0, int t1, hipStream_t s) {
   const int ntasks = t1 - t0;
   if (ntasks <= 0) return hipSuccess;
-  const int vw = row_width(N, ntasks);
+  const int vw = row_width(N, p.K, sizeof(TB), ntasks);
   const int nC = (N + 64 * vw - 1) / (64 * vw);
   const int64_t blocks = ((int64_t)ntasks * nC + 3) / 4;
   if (blocks > INT32_MAX / 4) return hipErrorInvalidValue;
@@ -231,7 +243,7 @@ hipError_t launch_sparse_rows(const SpmmPlanDev& p, const TB* B, int64_t ldb, in
 template <typename TB>
 hipError_t launch_sparse_pieces(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc, bool vec,
                            int pc0, int pc1, float* ws, hipStream_t s) {
-  const int vw = row_width(N, (int64_t)(pc1 - pc0) * 4);
+  const int vw = row_width(N, p.K, sizeof(TB), (int64_t)(pc1 - pc0) * 4);
   const int nC = (N + 64 * vw - 1) / (64 * vw);
   const int64_t blocks = (int64_t)(pc1 - pc0) * nC;
   if (blocks > INT32_MAX) return hipErrorInvalidValue;

@@ -89,3 +89,18 @@ def test_b_beyond_32_bit_offsets(cuda, dtype):
         B.copy_(torch.randn(K, N, device=cuda))
         print("wide B", N, dtype, flush=True)
         _check(A, B, plan.run_spmm(B))
+
+
+@pytest.mark.parametrize("K", [131072, 131073])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_columns_per_lane_on_both_sides_of_the_b_size_rule(cuda, K, dtype):
+    A = _matrix(K, 5, [40] * 1100 + [300, 700, 5000])
+    plan = _plan(A)
+    g = torch.Generator(device=cuda)
+    g.manual_seed(K)
+    B = torch.randn(K, 130, device=cuda, generator=g).to(getattr(torch, dtype))
+    print("rows", K, dtype, flush=True)
+    _check(A, B, plan.run_spmm(B))
+    once, again = plan.run_spmm(B, deterministic=True), plan.run_spmm(B, deterministic=True)
+    _check(A, B, once)
+    assert torch.equal(once, again)
