@@ -241,6 +241,26 @@ hipError_t launch_csr_sddmm_f32(int M, int nnz, int Kf, const int32_t* indptr,
 // FP32 on B's exact values (FP64 sums for hub rows and pieces).
 // ---------------------------------------------------------------------------
 
+// The plan arrays that the B-stationary kernel and its tail of sparse rows read:
+// what those launches pass of a plan.  The size of a launch's arguments shows in
+// its time.  With the whole SpmmPlanDev among them the kernel's were 864 bytes,
+// and two fields more in that structure (880 bytes, the kernel's instructions the
+// same) made the block-pruned layer at N = 4096 slower, 12.97 -> 13.13 us a pass;
+// with these arrays alone (464 bytes) it takes 13.00.
+struct WindowArrays {
+  int32_t W, W_tc;
+  const int32_t *win_rows, *tc_cols;
+  const void* tc_vals;
+  const int2* sp_ent;
+  const int32_t *res_ptr, *res_cols;
+  const float* res_vals;
+};
+static_assert(sizeof(WindowArrays) == 64, "arguments of the B-stationary launch: see above");
+
+static WindowArrays window_arrays(const SpmmPlanDev& p) {
+  return {p.W, p.W_tc, p.win_rows, p.tc_cols, p.tc_vals, p.sp_ent, p.res_ptr, p.res_cols, p.res_vals};
+}
+
 // Output rows of the 4 slots a lane group stores.  Loaded before any of the
 // window's C stores: vector-memory counters complete in issue order on
 // CDNA, so a load issued after a store would wait for it.
@@ -248,7 +268,7 @@ struct SlotRows {
   int row[4];
 };
 
-__device__ __forceinline__ SlotRows load_rows(const SpmmPlanDev& p, int slot0) {
+__device__ __forceinline__ SlotRows load_rows(const WindowArrays& p, int slot0) {
   SlotRows sr;
 #pragma unroll
   for (int i = 0; i < 4; ++i) sr.row[i] = p.win_rows[slot0 + i];
@@ -277,7 +297,7 @@ __device__ __forceinline__ void store_window(float* __restrict__ C, int64_t ldc,
 // over the four groups.  Rows with more than kHubNnz sparse nonzeros sum with
 // Neumaier compensation.
 template <typename TB>
-__device__ __forceinline__ void sparse_split_wave(const SpmmPlanDev& p, const TB* __restrict__ B, int64_t ldb,
+__device__ __forceinline__ void sparse_split_wave(const WindowArrays& p, const TB* __restrict__ B, int64_t ldb,
                                                   int N, float* __restrict__ C, int64_t ldc, int nC, bool vec,
                                                   int64_t wave) {
   const int lane = threadIdx.x & 63;
@@ -337,7 +357,7 @@ __device__ __forceinline__ void sparse_split_wave(const SpmmPlanDev& p, const TB
 }
 
 template <typename TB>
-__global__ __launch_bounds__(256) void hyb_spmm_sparse_split_kernel(SpmmPlanDev p, const TB* __restrict__ B,
+__global__ __launch_bounds__(256) void hyb_spmm_sparse_split_kernel(WindowArrays p, const TB* __restrict__ B,
                                                                     int64_t ldb, int N, float* __restrict__ C,
                                                                     int64_t ldc, int nC, bool vec) {
   with_vec(vec, [&](auto V) {
@@ -499,7 +519,7 @@ struct TrChunk {
   bool sc;
 };
 
-__device__ __forceinline__ TrChunk load_tr_chunk(const SpmmPlanDev& p, int c, int cidx, int lane, bool sc) {
+__device__ __forceinline__ TrChunk load_tr_chunk(const WindowArrays& p, int c, int cidx, int lane, bool sc) {
   TrChunk r;
   const int32_t* cp = p.tc_cols + (int64_t)c * 32 + cidx;
   r.k0 = cp[0];
@@ -547,7 +567,7 @@ __device__ __forceinline__ void tr_chunk_mfma(lds_u8* lds, int cst, const TrChun
 }
 
 // Rows of the lane group's 4 window slots.
-__device__ __forceinline__ SlotRows load_win(const SpmmPlanDev& p, int slot0) { return load_rows(p, slot0); }
+__device__ __forceinline__ SlotRows load_win(const WindowArrays& p, int slot0) { return load_rows(p, slot0); }
 
 // One round of a window's sparse part (kMixed plans): e holds the round's
 // entry of slot 4g + (lane & 3) (column, value bits); lane (g, j) adds
@@ -637,7 +657,7 @@ __device__ __forceinline__ void store_window_lds(float* __restrict__ C, int64_t 
 }
 
 template <typename TB, bool kMixed, int kStore, bool kSc>
-__device__ __forceinline__ void lds_item(const SpmmPlanDev& p, const int32_t* __restrict__ tc_ptr,
+__device__ __forceinline__ void lds_item(const WindowArrays& p, const int32_t* __restrict__ tc_ptr,
                                          const int32_t* __restrict__ sp_off, const uint32_t* __restrict__ tc_kind,
                                          const int32_t* __restrict__ win_r0, const int4* __restrict__ units,
                                          const TB* __restrict__ B, int64_t ldb, int N, float* __restrict__ C,
@@ -818,7 +838,7 @@ __device__ __forceinline__ void lds_item(const SpmmPlanDev& p, const int32_t* __
 // each XCD, which holds the fewest items when a range does not divide evenly;
 // one-item launches add tail blocks past the items when CUs are free.
 template <bool kLoop, typename TB, bool kMixed, int kStore>
-__global__ __launch_bounds__(kLdsThreads) void hyb_spmm_lds_bf16_kernel(SpmmPlanDev p,
+__global__ __launch_bounds__(kLdsThreads) void hyb_spmm_lds_bf16_kernel(WindowArrays p,
                                                                         const int32_t* __restrict__ tc_ptr,
                                                                         const int32_t* __restrict__ sp_off,
                                                                         const uint32_t* __restrict__ tc_kind,
@@ -979,7 +999,7 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
     const int cbytes = p.M > 0 && c_extent < ((int64_t)1 << 31) ? (int)c_extent : 0;
 #define STILE_LDS_LAUNCH1(LOOP, MIX, VEC)                                                                    \
   hipLaunchKernelGGL((hyb_spmm_lds_bf16_kernel<LOOP, TB, MIX, VEC>), dim3(grid), dim3(kLdsThreads), lds_bytes, s, \
-                     p,                                                                                        \
+                     window_arrays(p),                                                                         \
                      p.tc_ptr, p.sp_off, p.tc_kind, p.win_r0, units, B, ldb, N, C, ldc, nC, (int)items, vec, vec16, \
                      cbytes, xr, LOOP && xcd, tail_blocks, tail_tasks)
 #define STILE_LDS_LAUNCH(LOOP, MIX)                \
@@ -1013,8 +1033,8 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
   const bool split = so_left > 0 && so_left * nC / 4 < 4096 && p.nnz_sparse_only >= 8 * so_left;
   if (split) {
     const int64_t blocks = (so_rows * nC + 3) / 4;
-    hipLaunchKernelGGL(hyb_spmm_sparse_split_kernel<TB>, dim3((unsigned)blocks), dim3(256), 0, s, p, B, ldb, N, C,
-                       ldc, nC, vec);
+    hipLaunchKernelGGL(hyb_spmm_sparse_split_kernel<TB>, dim3((unsigned)blocks), dim3(256), 0, s,
+                       window_arrays(p), B, ldb, N, C, ldc, nC, vec);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
