@@ -214,6 +214,8 @@ def _split_k_tn(H, G, slab_rows=16384):
     179 / 56, 64 182 / 146, 128 334 / 299, 256 1140 / 953; M = 2^18 71 / 51, 71 /
     47, 101 / 104, 326 / 264; M = 2^17 55 / 55, 55 / 92, 65 / 66, 165 / 139; M =
     2^16 49 / 56, 48 / 90, 48 / 98, 92 / 115."""
+    if H.dim() != 2 or G.dim() != 2:  # a vector of weights
+        return H.t() @ G
     M = H.shape[0]
     slabs = H.dtype == G.dtype == torch.float32 and M % slab_rows == 0 and M >= 4 * slab_rows
     beaten = slabs and (M >= 1 << 18 or M * H.shape[1] * G.shape[1] >= 1 << 33)
