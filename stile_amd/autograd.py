@@ -186,13 +186,26 @@ def sddmm(op, X, Y):
 _TALL_ROWS = 4096
 
 
+def _own_memory(t):
+    """True for a tensor whose data_ptr is its values: no subclass, no wrapper of
+    a function transform (vmap's batched tensors have the type torch.Tensor and
+    one sample's shape, but no memory of their own), and no negation left to do."""
+    if type(t) is not torch.Tensor or t.is_neg():
+        return False
+    try:
+        t.data_ptr()
+    except RuntimeError:
+        return False
+    return True
+
+
 def _tall_kernel_fits(H, G):
     """True where the library's own H^T G runs instead of a GEMM: plain float32
-    device tensors, outside tracing and outside a backward pass that is itself
-    differentiated, with many more rows than output entries per side (a GEMM has
-    one workgroup per output tile and a few splits of the rows; measured at
-    M = 32768, F = Fg = 256: 138 us against 56)."""
-    if not (type(H) is type(G) is torch.Tensor and H.is_cuda and G.is_cuda and H.dtype == G.dtype == torch.float32):
+    device matrices, outside tracing and outside a backward
+    pass that is itself differentiated, with many more rows than output entries
+    per side (a GEMM has one workgroup per output tile and a few splits of the
+    rows; measured at M = 32768, F = Fg = 256: 138 us against 56)."""
+    if not (H.is_cuda and G.is_cuda and H.dtype == G.dtype == torch.float32 and _own_memory(H) and _own_memory(G)):
         return False
     M, F, Fg = H.shape[0], H.shape[1], G.shape[1]
     span = (1 << 32) - (1 << 20)

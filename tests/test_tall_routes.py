@@ -4,6 +4,7 @@ weights): they take the products of torch, on every device."""
 import pytest
 import torch
 
+from stile_amd import autograd
 from stile_amd.autograd import tall_matmul
 
 M, F, FG = 4100, 12, 9  # rows beyond those from which the library's kernel runs
@@ -24,6 +25,30 @@ def _check(H, G, got):
     assert torch.all((got.detach().cpu().double() - H64.t() @ G64).abs() <= bound)
 
 
+def _batched(dev):
+    H, W, dY = _operands(dev)
+    dW, = torch.autograd.grad(tall_matmul(H, W), W, dY, is_grads_batched=True)
+    assert dW.shape == (4, F, FG)
+    for i in range(4):
+        _check(H, dY[i], dW[i])
+
+
+def _vmap(dev):
+    H, W, dY = _operands(dev)
+    y = tall_matmul(H, W)
+    dW = torch.vmap(lambda d: torch.autograd.grad(y, W, d, retain_graph=True)[0])(dY)
+    for i in range(4):
+        _check(H, dY[i], dW[i])
+
+
+def _negated(dev):
+    H, W, dY = _operands(dev)
+    d = torch.complex(dY[0], dY[1]).conj().imag
+    assert d.is_neg()
+    dW, = torch.autograd.grad(tall_matmul(H, W), W, d)
+    _check(H, -dY[1], dW)
+
+
 def _vector(dev):
     H, _, dY = _operands(dev)
     w = torch.randn(F, device=dev, requires_grad=True)
@@ -32,7 +57,7 @@ def _vector(dev):
     _check(H, dY[0, :, :1], dw[:, None])
 
 
-ROUTES = [_vector]
+ROUTES = [_batched, _vmap, _negated, _vector]
 
 
 @pytest.mark.parametrize("route", ROUTES)
@@ -45,3 +70,19 @@ def test_on_the_cpu(route):
 def test_on_the_gpu(cuda, route):
     print("tall route", route.__name__, flush=True)
     route(cuda)
+
+
+@pytest.mark.parametrize("route", [_batched, _vmap, _negated])
+def test_operands_without_memory_of_their_own_are_told_apart(monkeypatch, route):
+    seen = []
+
+    def spy(H, G):
+        seen.append(autograd._own_memory(G))
+        return H.t() @ G
+
+    monkeypatch.setattr(autograd, "_split_k_tn", spy)
+    route("cpu")
+    assert seen and not any(seen)
+    H, W, dY = _operands("cpu")
+    torch.autograd.grad(tall_matmul(H, W), W, dY[0])
+    assert seen[-1]
