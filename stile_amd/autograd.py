@@ -22,6 +22,7 @@ import os
 import numpy as np
 import scipy.sparse
 import torch
+from torch.autograd import forward_ad
 
 from . import _native, api
 
@@ -189,14 +190,15 @@ _TALL_ROWS = 4096
 def _own_memory(t):
     """True for a tensor whose data_ptr is its values: no subclass, no wrapper of
     a function transform (vmap's batched tensors have the type torch.Tensor and
-    one sample's shape, but no memory of their own), and no negation left to do."""
+    one sample's shape, but no memory of their own), no negation left to do, no
+    forward-mode tangent that a raw pointer would lose."""
     if type(t) is not torch.Tensor or t.is_neg():
         return False
     try:
         t.data_ptr()
     except RuntimeError:
         return False
-    return True
+    return forward_ad.unpack_dual(t).tangent is None
 
 
 def _tall_kernel_fits(H, G):

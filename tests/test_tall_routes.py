@@ -3,6 +3,7 @@ memory (batched by vmap, forward-mode duals, lazily negated views, a vector of
 weights): they take the products of torch, on every device."""
 import pytest
 import torch
+from torch.autograd import forward_ad
 
 from stile_amd import autograd
 from stile_amd.autograd import tall_matmul
@@ -41,6 +42,17 @@ def _vmap(dev):
         _check(H, dY[i], dW[i])
 
 
+def _dual(dev):
+    H, W, dY = _operands(dev)
+    y = tall_matmul(H, W)
+    with forward_ad.dual_level():
+        dW, = torch.autograd.grad(y, W, forward_ad.make_dual(dY[0], dY[1]))
+        got = forward_ad.unpack_dual(dW)
+        _check(H, dY[0], got.primal)
+        assert got.tangent is not None
+        _check(H, dY[1], got.tangent)
+
+
 def _negated(dev):
     H, W, dY = _operands(dev)
     d = torch.complex(dY[0], dY[1]).conj().imag
@@ -57,7 +69,7 @@ def _vector(dev):
     _check(H, dY[0, :, :1], dw[:, None])
 
 
-ROUTES = [_batched, _vmap, _negated, _vector]
+ROUTES = [_batched, _vmap, _dual, _negated, _vector]
 
 
 @pytest.mark.parametrize("route", ROUTES)
@@ -72,7 +84,7 @@ def test_on_the_gpu(cuda, route):
     route(cuda)
 
 
-@pytest.mark.parametrize("route", [_batched, _vmap, _negated])
+@pytest.mark.parametrize("route", [_batched, _vmap, _dual, _negated])
 def test_operands_without_memory_of_their_own_are_told_apart(monkeypatch, route):
     seen = []
 
