@@ -23,6 +23,7 @@ import numpy as np
 import scipy.sparse
 import torch
 from torch.autograd import forward_ad
+from torch.utils._python_dispatch import is_in_torch_dispatch_mode
 
 from . import _native, api
 
@@ -203,7 +204,7 @@ def _own_memory(t):
 
 def _tall_kernel_fits(H, G):
     """True where the library's own H^T G runs instead of a GEMM: plain float32
-    device matrices, outside tracing and outside a backward
+    device matrices, outside tracing and dispatch modes and outside a backward
     pass that is itself differentiated, with many more rows than output entries
     per side (a GEMM has one workgroup per output tile and a few splits of the
     rows; measured at M = 32768, F = Fg = 256: 138 us against 56)."""
@@ -213,7 +214,8 @@ def _tall_kernel_fits(H, G):
     span = (1 << 32) - (1 << 20)
     return (M >= _TALL_ROWS and 0 < F <= M // 32 and 0 < Fg <= M // 32 and F * Fg <= 1 << 20
             and 4 * M * max(H.stride(0), F) < span and 4 * M * max(G.stride(0), Fg) < span
-            and not torch.is_grad_enabled() and not torch.compiler.is_compiling())
+            and not torch.is_grad_enabled() and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and not is_in_torch_dispatch_mode())
 
 
 def _split_k_tn(H, G, slab_rows=16384):

@@ -4,6 +4,7 @@ weights): they take the products of torch, on every device."""
 import pytest
 import torch
 from torch.autograd import forward_ad
+from torch.utils.flop_counter import FlopCounterMode
 
 from stile_amd import autograd
 from stile_amd.autograd import tall_matmul
@@ -69,7 +70,15 @@ def _vector(dev):
     _check(H, dY[0, :, :1], dw[:, None])
 
 
-ROUTES = [_batched, _vmap, _dual, _negated, _vector]
+def _counted(dev):
+    H, W, dY = _operands(dev)
+    with FlopCounterMode(display=False) as mode:
+        dW, = torch.autograd.grad(tall_matmul(H, W), W, dY[0])
+    assert mode.get_total_flops() == 2 * (2 * M * F * FG)
+    _check(H, dY[0], dW)
+
+
+ROUTES = [_batched, _vmap, _dual, _negated, _vector, _counted]
 
 
 @pytest.mark.parametrize("route", ROUTES)
