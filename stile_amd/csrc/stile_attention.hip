@@ -325,6 +325,13 @@ __global__ __launch_bounds__(64, 3) void attention_fused_kernel(SpmmPlanDev p, A
         sval[u] = on[u] ? dot : -INFINITY;
         m_run = fmaxf(m_run, sval[u]);
       }
+      // V rows read for entries past a row's end weigh nothing, whatever they hold
+      // (0 times an infinity or a NaN is a NaN)
+      if (!__all(on[kAttBatch - 1])) {
+#pragma unroll
+        for (int u = 0; u < kAttBatch; ++u)
+          if (!on[u]) va[u] = vb[u] = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
+      }
       auto prob = [&](float x, float mx) { return x == -INFINITY ? 0.f : __expf((x - mx) * scale); };
       if (__all(m_run == ms)) {
         // no row's maximum moved: entries two at a time (v_dot2_f32_bf16)
