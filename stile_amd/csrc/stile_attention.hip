@@ -385,8 +385,10 @@ hipError_t launch_attention(const SpmmPlanDev& p, const AttOrder& ord, const voi
   if (p.W == 0) return hipSuccess;
   int longest = 0;
   for (int x = 0; x < kXcds; ++x) longest = max(longest, ord.start[x + 1] - ord.start[x]);
-  // 32-bit row offsets from 24-bit products: up to 2^24 rows and 4 GiB
-  const bool small = p.M < (1 << 24) && ld < (1 << 23) && (int64_t)p.M * ld * 2 < ((int64_t)1 << 32);
+  // 32-bit row offsets from 24-bit products: up to 2^24 rows and 4 GiB (of Q: M,
+  // of K and V: K, equal in attention plans)
+  const int64_t rows = max(p.M, p.K);
+  const bool small = rows < (1 << 24) && ld < (1 << 23) && rows * ld * 2 < ((int64_t)1 << 32);
   const auto kernel = small ? attention_fused_kernel<true> : attention_fused_kernel<false>;
   hipLaunchKernelGGL(kernel, dim3((unsigned)(longest * kXcds)), dim3(64), 0, s, p, ord,
                      static_cast<const __bf16*>(Q), static_cast<const __bf16*>(K), static_cast<const __bf16*>(V),

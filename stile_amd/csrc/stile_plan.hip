@@ -1079,7 +1079,8 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   const size_t o_r0 = lay.add(win_r0.size() * 4);
   std::vector<int32_t> att_win;
   stile::AttOrder att{};
-  if (bd.want_mask) attention_order(bd.win_rows, tc_ptr, res_ptr, att_win, att.start);
+  // (a plan without dense chunks runs attention too, however it was made)
+  if (bd.want_mask || tc_ptr[W] == 0) attention_order(bd.win_rows, tc_ptr, res_ptr, att_win, att.start);
   const size_t o_rtask = lay.add(row_tasks.size() * 4);
   const size_t o_att = lay.add(att_win.size() * 4);
   HostBlob blob;
