@@ -117,7 +117,8 @@ __global__ __launch_bounds__(64, 3) void attention_fused_kernel(SpmmPlanDev p, A
                                                                 const __bf16* __restrict__ Qm,
                                                                 const __bf16* __restrict__ Km,
                                                                 const __bf16* __restrict__ Vm, int64_t ld,
-                                                                float scale, float* __restrict__ out, int64_t ldo) {
+                                                                float scale, float* __restrict__ out, int64_t ldo,
+                                                                int first) {
   // the chunk's 32 K and 32 V rows; after them the sums on their way to the sparse part
   __shared__ __align__(16) unsigned char stage[64 * kAttVRow];
   static_assert(64 * kAttVRow >= 4 * 16 * kAttOStride);
@@ -130,7 +131,7 @@ __global__ __launch_bounds__(64, 3) void attention_fused_kernel(SpmmPlanDev p, A
       o0 = ord.start[i];
       o1 = ord.start[i + 1];
     }
-  const int oi = o0 + (int)(blockIdx.x / kXcds);
+  const int oi = o0 + first + (int)(blockIdx.x / kXcds);
   if (oi >= o1) return;
   const int w = __builtin_amdgcn_readfirstlane(ord.win[oi]);
   lds_u8* const vt = (lds_u8*)stage;
@@ -390,10 +391,15 @@ hipError_t launch_attention(const SpmmPlanDev& p, const AttOrder& ord, const voi
   const int64_t rows = max(p.M, p.K);
   const bool small = rows < (1 << 24) && ld < (1 << 23) && rows * ld * 2 < ((int64_t)1 << 32);
   const auto kernel = small ? attention_fused_kernel<true> : attention_fused_kernel<false>;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(longest * kXcds)), dim3(64), 0, s, p, ord,
-                     static_cast<const __bf16*>(Q), static_cast<const __bf16*>(K), static_cast<const __bf16*>(V),
-                     ld, scale, out, ldo);
-  return hipGetLastError();
+  constexpr int kMost = (int)(max_blocks(64) / kXcds);
+  hipError_t e = hipSuccess;
+  for (int first = 0; first < longest && e == hipSuccess; first += kMost) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(min(kMost, longest - first) * kXcds)), dim3(64), 0, s, p, ord,
+                       static_cast<const __bf16*>(Q), static_cast<const __bf16*>(K), static_cast<const __bf16*>(V),
+                       ld, scale, out, ldo, first);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 }  // namespace stile

@@ -199,6 +199,10 @@ struct SddmmPlanDev {
   const int32_t* blk_out;
 };
 
+// Workgroups of one launch: a grid dimension holds fewer than 2^32 threads, larger
+// work goes in several launches.
+constexpr int64_t max_blocks(int threads) { return (((int64_t)1 << 32) - 1) / threads; }
+
 // Kernel launchers (stile_kernels.hip).  All return hipError_t of the launch.
 // Compute units of the current device (queried once per device).
 int device_cus();

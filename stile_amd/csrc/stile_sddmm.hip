@@ -221,10 +221,9 @@ hipError_t launch_hyb_sddmm(const SddmmPlanDev& p, const float* X,
   const int epw = 64 / lpe * kSddmmU;
   const int64_t waves1d = ((int64_t)p.n1d + epw - 1) / epw;
   const int64_t blocks1d = (waves1d + 3) / 4;
-  const int bpb = Kf > kSharedKf ? 1 : 4;
+  const int bpb = Kf > kSharedKf && blocks1d + p.nblk <= max_blocks(256) ? 1 : 4;
   const int64_t blocks = blocks1d + ((int64_t)p.nblk + bpb - 1) / bpb;
   if (blocks == 0) return hipSuccess;
-  if (blocks > INT32_MAX) return hipErrorInvalidValue;
   auto small = [&](int64_t rows, int64_t ld) {
     return rows <= (1 << 24) && ld < (1 << 22) && ((rows - 1) * ld + Kf) * 4 < ((int64_t)1 << 32);
   };

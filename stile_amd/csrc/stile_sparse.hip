@@ -229,15 +229,19 @@ hipError_t launch_sparse_rows(const SpmmPlanDev& p, const TB* B, int64_t ldb, in
   if (ntasks <= 0) return hipSuccess;
   const int vw = row_width(N, p.K, sizeof(TB), ntasks);
   const int nC = (N + 64 * vw - 1) / (64 * vw);
-  const int64_t blocks = ((int64_t)ntasks * nC + 3) / 4;
-  if (blocks > INT32_MAX / 4) return hipErrorInvalidValue;
   const uint32_t bytes = b_bytes<TB>(p.K, ldb, N);
-  with_width(vw, vec, bytes > 0, [&](auto w, auto v, auto u) {
-    hipLaunchKernelGGL((hyb_spmm_rows_kernel<TB, decltype(w)::value, decltype(v)::value, decltype(u)::value>),
-                       dim3((unsigned)blocks), dim3(256), 0, s, p.row_tasks + t0, ntasks, p.res_ptr, p.res_cols,
-                       p.res_vals, p.win_rows, B, ldb, bytes, N, C, ldc, nC);
-  });
-  return hipGetLastError();
+  hipError_t e = hipSuccess;
+  const int per = (int)std::max<int64_t>(1, std::min<int64_t>(ntasks, max_blocks(256) * 4 / nC));
+  for (int a = t0; a < t1 && e == hipSuccess; a += std::min(per, t1 - a)) {
+    const int n = std::min(per, t1 - a);
+    with_width(vw, vec, bytes > 0, [&](auto w, auto v, auto u) {
+      hipLaunchKernelGGL((hyb_spmm_rows_kernel<TB, decltype(w)::value, decltype(v)::value, decltype(u)::value>),
+                         dim3((unsigned)(((int64_t)n * nC + 3) / 4)), dim3(256), 0, s, p.row_tasks + a, n, p.res_ptr,
+                         p.res_cols, p.res_vals, p.win_rows, B, ldb, bytes, N, C, ldc, nC);
+    });
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 template <typename TB>
@@ -245,26 +249,33 @@ hipError_t launch_sparse_pieces(const SpmmPlanDev& p, const TB* B, int64_t ldb, 
                            int pc0, int pc1, float* ws, hipStream_t s) {
   const int vw = row_width(N, p.K, sizeof(TB), (int64_t)(pc1 - pc0) * 4);
   const int nC = (N + 64 * vw - 1) / (64 * vw);
-  const int64_t blocks = (int64_t)(pc1 - pc0) * nC;
-  if (blocks > INT32_MAX) return hipErrorInvalidValue;
   const uint32_t bytes = b_bytes<TB>(p.K, ldb, N);
-  with_width(vw, vec, bytes > 0, [&](auto w, auto v, auto u) {
-    hipLaunchKernelGGL((hyb_spmm_pieces_kernel<TB, decltype(w)::value, decltype(v)::value, decltype(u)::value>),
-                       dim3((unsigned)blocks), dim3(256), 0, s, p.piece_exec, p.piece_row, p.piece_beg, p.piece_end,
-                       pc0, pc1 - pc0, p.res_cols, p.res_vals, B, ldb, bytes, N, C, ldc, ws);
-  });
-  return hipGetLastError();
+  hipError_t e = hipSuccess;
+  const int per = (int)std::max<int64_t>(1, std::min<int64_t>(pc1 - pc0, max_blocks(256) / nC));
+  for (int a = pc0; a < pc1 && e == hipSuccess; a += std::min(per, pc1 - a)) {
+    const int n = std::min(per, pc1 - a);
+    with_width(vw, vec, bytes > 0, [&](auto w, auto v, auto u) {
+      hipLaunchKernelGGL((hyb_spmm_pieces_kernel<TB, decltype(w)::value, decltype(v)::value, decltype(u)::value>),
+                         dim3((unsigned)((int64_t)n * nC)), dim3(256), 0, s, p.piece_exec, p.piece_row, p.piece_beg,
+                         p.piece_end, a, n, p.res_cols, p.res_vals, B, ldb, bytes, N, C, ldc, ws);
+    });
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 hipError_t launch_piece_reduce(const SpmmPlanDev& p, int N, float* C, int64_t ldc, bool vec, int sr0, const float* ws,
                                hipStream_t s) {
   const int nC = (N + 63) / 64;
-  const int64_t blocks = (int64_t)(p.nsrows - sr0) * nC;
-  if (blocks <= 0) return hipSuccess;
-  if (blocks > INT32_MAX) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(hyb_spmm_piece_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, s, p, N, C, ldc, nC, vec, sr0,
-                     ws);
-  return hipGetLastError();
+  hipError_t e = hipSuccess;
+  const int per = (int)std::max<int64_t>(1, std::min<int64_t>(p.nsrows, max_blocks(256) / nC));
+  for (int a = sr0; a < p.nsrows && e == hipSuccess; a += std::min(per, p.nsrows - a)) {
+    const int n = std::min(per, p.nsrows - a);
+    hipLaunchKernelGGL(hyb_spmm_piece_reduce_kernel, dim3((unsigned)((int64_t)n * nC)), dim3(256), 0, s, p, N, C, ldc,
+                       nC, vec, a, ws);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 template hipError_t launch_sparse_rows<float>(const SpmmPlanDev&, const float*, int64_t, int, float*, int64_t, bool, int,

@@ -324,23 +324,25 @@ __device__ __forceinline__ void stream_window(const StreamArrays& A, const int32
 
 // Blocks [0, (n_parts + W_big - W_huge) * nC2) each run one (part of a huge
 // window or other big window, 32 columns) on all its waves; the next ones run
-// the (W_tc - W_big) * nC (window, 64 columns) on nw waves each.  Parts add into C with atomicAdd (C rows zeroed before),
-// or, with ws (deterministic mode), store to ws[part][16][N]; the first part of
-// a window brings its sparse part.
+// the (W_tc - W_big) * nC (window, 64 columns) on nw waves each.  The launch runs
+// them from block0 on.  Parts add into C with atomicAdd (C rows zeroed before), or,
+// with ws (deterministic mode), store to ws[part][16][N]; the first part of a
+// window brings its sparse part.
 template <int MODE, typename TB, bool kVec, bool kBuf>
 __global__ __launch_bounds__(kStreamWaves * 64, 4) void hyb_spmm_stream_kernel(
     SpmmPlanDev p, const int32_t* __restrict__ res_ptr, const int32_t* __restrict__ res_cols,
     const float* __restrict__ res_vals, const TB* __restrict__ B, int64_t ldb, uint32_t bbytes, int N,
-    float* __restrict__ C, int64_t ldc, int nC, int nC2, int nw, float* __restrict__ ws) {
+    float* __restrict__ C, int64_t ldc, int nC, int nC2, int nw, float* __restrict__ ws, int block0) {
   extern __shared__ float4 stream_lds[];
   float* lds = reinterpret_cast<float*>(stream_lds);
   const StreamArrays A{p.tc_ptr, p.tc_cols, p.res_ptr, p.res_cols, p.win_rows, p.tc_vals, p.tc_scale, p.res_vals};
+  const int block = block0 + (int)blockIdx.x;
   const int big = (p.n_parts + p.W_big - p.W_huge) * nC2;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bool fold = p.fold_mix != 0;
   auto has_sparse = [&](int w) { return fold && res_ptr[w * 16] < res_ptr[w * 16 + 16]; };
-  if ((int)blockIdx.x < big) {
-    const int i = (int)blockIdx.x / nC2, n0 = ((int)blockIdx.x - i * nC2) * 32;
+  if (block < big) {
+    const int i = block / nC2, n0 = (block - i * nC2) * 32;
     if (i < p.n_parts) {
       const int w = p.part_win[i];
       stream_window<MODE, TB, 2, kVec, kBuf>(A, res_ptr, res_cols, res_vals, B, ldb, bbytes, N, C, ldc, w, n0,
@@ -357,7 +359,7 @@ __global__ __launch_bounds__(kStreamWaves * 64, 4) void hyb_spmm_stream_kernel(
   // kStreamWaves / nw windows side by side; the workgroup's last ones may have no
   // window left and only meet the others at the barrier
   const int sub = wv / nw;
-  const int job = ((int)blockIdx.x - big) * (kStreamWaves / nw) + sub;
+  const int job = (block - big) * (kStreamWaves / nw) + sub;
   const int i = job / nC, n0 = (job - i * nC) * 64;
   const int w = p.W_big + i;
   if (w < p.W_tc)
@@ -417,10 +419,11 @@ hipError_t launch_stream(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, 
   uint32_t bytes = b_bytes<TB>(p.K, ldb, N);
   if (p.K > (1 << 24) || ldb * (int64_t)sizeof(TB) >= (1 << 24)) bytes = 0;
   const size_t lds = (size_t)(kStreamWaves + per) * 16 * 64 * 4;
+  int64_t b0 = 0, n = 0;
   auto go = [&](auto mode, auto v, auto u) {
     hipLaunchKernelGGL((hyb_spmm_stream_kernel<decltype(mode)::value, TB, decltype(v)::value, decltype(u)::value>),
-                       dim3((unsigned)blocks), dim3(kStreamWaves * 64), lds, s, p, p.res_ptr, p.res_cols, p.res_vals, B, ldb,
-                       bytes, N, C, ldc, nC, nC2, nw, ws);
+                       dim3((unsigned)n), dim3(kStreamWaves * 64), lds, s, p, p.res_ptr, p.res_cols, p.res_vals, B,
+                       ldb, bytes, N, C, ldc, nC, nC2, nw, ws, (int)b0);
   };
   auto by_layout = [&](auto mode) {
     if (bytes > 0 && vec)
@@ -430,14 +433,18 @@ hipError_t launch_stream(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, 
     else
       go(mode, std::false_type{}, std::false_type{});
   };
-  if (p.blk_dtype == 1)
-    by_layout(std::integral_constant<int, 1>{});
-  else if (p.blk_dtype == 2)
-    by_layout(std::integral_constant<int, 2>{});
-  else
-    by_layout(std::integral_constant<int, 0>{});
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  hipError_t e = hipSuccess;
+  for (; b0 < blocks; b0 += n) {
+    n = std::min(blocks - b0, max_blocks(kStreamWaves * 64));
+    if (p.blk_dtype == 1)
+      by_layout(std::integral_constant<int, 1>{});
+    else if (p.blk_dtype == 2)
+      by_layout(std::integral_constant<int, 2>{});
+    else
+      by_layout(std::integral_constant<int, 0>{});
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   if (ws && p.W_huge > 0) {
     const int64_t waves = (int64_t)p.W_huge * nC;
     hipLaunchKernelGGL(hyb_spmm_part_reduce_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, p, N, C, ldc,

@@ -1,0 +1,66 @@
+"""Products whose workgroups are more than one launch takes (a grid dimension holds
+fewer than 2^32 threads): few rows and 2^22 columns, so that the matrices stay small.
+
+Every entry of C is written; columns at the ends, at the cuts and between are
+compared with FP64, per element within (n + 2) 2^-24 sum|a||b| for rows of n
+entries (n products, rounded and added in FP32 in some order)."""
+import numpy as np
+import pytest
+import scipy.sparse
+import torch
+
+from stile_amd import _native, api
+
+pytestmark = pytest.mark.gpu
+
+N = 1 << 22
+
+
+def _run(cuda, A, search, deterministic):
+    opts = api.options_for("float32")
+    setattr(opts, search, True)
+    plan = _native.Plan.spmm(api.spmm_pack(A, opts)[0], "float32")
+    g = torch.Generator(device=cuda)
+    g.manual_seed(1)
+    B = torch.randn(A.shape[1], N, device=cuda, generator=g)
+    C = torch.full((A.shape[0], N), float("nan"), device=cuda)
+    print("launch limits", A.shape, A.nnz, search, deterministic, plan.info(), flush=True)
+    plan.run_spmm(B, C, deterministic=deterministic)
+    for r in range(0, A.shape[0], 128):
+        assert not torch.isnan(C[r:r + 128]).any()
+    cols = torch.cat([torch.arange(130), torch.arange(N // 2 - 70, N // 2 + 70), torch.arange(N - 130, N),
+                      torch.randint(N, (200,), generator=torch.Generator().manual_seed(2))]).to(cuda)
+    A64, B64 = torch.from_numpy(A.toarray()).to(cuda).double(), B[:, cols].double()
+    bound = (np.diff(A.indptr).max() + 2) * 2.0 ** -24 * (A64.abs() @ B64.abs())
+    assert torch.all((C[:, cols].double() - A64 @ B64).abs() <= bound)
+    return plan.info()
+
+
+@pytest.fixture(autouse=True)
+def _free(cuda):
+    yield
+    torch.cuda.empty_cache()
+
+
+def _full(M, K):
+    return scipy.sparse.csr_matrix(np.random.default_rng(M + K).standard_normal((M, K)).astype(np.float32))
+
+
+def test_sparse_rows(cuda):
+    # 2048 wave tasks of 64 entries, 32768 column chunks of 128
+    info = _run(cuda, _full(2048, 64), "only_ELL", False)
+    assert info["num_chunks"] == 0 and info["num_split"] == 0
+
+
+@pytest.mark.parametrize("deterministic", [False, True])
+def test_pieces_of_long_rows(cuda, deterministic):
+    # 512 pieces behind 256 rows' first 256 entries, 32768 column chunks of 128;
+    # the reduce kernel 256 rows of 65536 chunks of 64
+    info = _run(cuda, _full(256, 768), "only_ELL", deterministic)
+    assert info["num_split"] == 512
+
+
+def test_dense_windows(cuda):
+    # 128 windows of 6 chunks, a workgroup for each 64 of 2^22 columns
+    info = _run(cuda, _full(2048, 192), "only_TC", False)
+    assert info["sparse_nnz"] == 0 and info["num_chunks"] == 768
