@@ -207,7 +207,7 @@ __device__ __forceinline__ void stream_window(const StreamArrays& A, const int32
   static_assert(D >= 1);
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, j = lane & 15;
-  const int share = (c1 - c0 + nw - 1) / nw;
+  const int share = max((c1 - c0 + nw - 1) / nw, 1);  // (no chunks: see the kernel's last job)
   const int nd = (c1 - c0 + share - 1) / share;  // waves with a share
   const int a = min(c0 + wv * share, c1), b = min(a + share, c1);
   // Sparse entries of the window's slots: on the waves without chunks when they
@@ -356,18 +356,18 @@ __global__ __launch_bounds__(kStreamWaves * 64, 4) void hyb_spmm_stream_kernel(
     }
     return;
   }
-  // kStreamWaves / nw windows side by side; the workgroup's last ones may have no
-  // window left and only meet the others at the barrier
+  // kStreamWaves / nw windows side by side; a last workgroup with fewer left runs
+  // the spare waves on no chunks and columns from N on, so that every wave meets
+  // the others at the same barrier and stores nothing
   const int sub = wv / nw;
   const int job = (block - big) * (kStreamWaves / nw) + sub;
-  const int i = job / nC, n0 = (job - i * nC) * 64;
-  const int w = p.W_big + i;
-  if (w < p.W_tc)
-    stream_window<MODE, TB, 4, kVec, kBuf>(A, res_ptr, res_cols, res_vals, B, ldb, bbytes, N, C, ldc, w, n0,
-                                           p.tc_ptr[w], p.tc_ptr[w + 1], has_sparse(w), nullptr, false,
-                                           lds + sub * (nw + 1) * 16 * 64, wv - sub * nw, nw);
-  else
-    __syncthreads();
+  const int i = job / nC;
+  const bool live = p.W_big + i < p.W_tc;
+  const int w = live ? p.W_big + i : p.W_tc - 1, n0 = live ? (job - i * nC) * 64 : N;
+  const int c0 = p.tc_ptr[w], c1 = live ? p.tc_ptr[w + 1] : c0;
+  stream_window<MODE, TB, 4, kVec, kBuf>(A, res_ptr, res_cols, res_vals, B, ldb, bbytes, N, C, ldc, w, n0, c0, c1,
+                                         live && has_sparse(w), nullptr, false, lds + sub * (nw + 1) * 16 * 64,
+                                         wv - sub * nw, nw);
 }
 
 // Deterministic mode: C rows of huge window w = sum of its parts' partial
