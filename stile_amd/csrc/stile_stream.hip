@@ -180,11 +180,13 @@ __device__ __forceinline__ void mfma_chunk(const ChunkA<MODE>& a, const ChunkB<T
   }
 }
 
-// Pointers of the plan the kernel reads with scalar loads between its stores.
+// What the kernel reads of a plan (a launch passes no more of it).
 struct StreamArrays {
-  const int32_t *tc_ptr, *tc_cols, *res_ptr, *res_cols, *win_rows;
+  const int32_t *tc_ptr, *tc_cols, *win_rows;
   const void* tc_vals;
-  const float *tc_scale, *res_vals;
+  const float* tc_scale;
+  const int32_t *part_win, *part_c0, *part_c1, *hw_p0;
+  int32_t W_tc, W_big, W_huge, n_parts, fold_mix;
 };
 
 // Registers for the chunks in flight (four waves per SIMD).  16-bit rows with
@@ -324,19 +326,18 @@ __device__ __forceinline__ void stream_window(const StreamArrays& A, const int32
 
 // Blocks [0, (n_parts + W_big - W_huge) * nC2) each run one (part of a huge
 // window or other big window, 32 columns) on all its waves; the next ones run
-// the (W_tc - W_big) * nC (window, 64 columns) on nw waves each.  The launch runs
-// them from block0 on.  Parts add into C with atomicAdd (C rows zeroed before), or,
-// with ws (deterministic mode), store to ws[part][16][N]; the first part of a
-// window brings its sparse part.
+// the (W_tc - W_big) * nC (window, 64 columns) on nw waves each.  Parts
+// add into C with atomicAdd (C rows zeroed before), or, with ws (deterministic
+// mode), store to ws[part][16][N]; the first part of a window brings its sparse
+// part.
 template <int MODE, typename TB, bool kVec, bool kBuf>
 __global__ __launch_bounds__(kStreamWaves * 64, 4) void hyb_spmm_stream_kernel(
-    SpmmPlanDev p, const int32_t* __restrict__ res_ptr, const int32_t* __restrict__ res_cols,
+    StreamArrays p, const int32_t* __restrict__ res_ptr, const int32_t* __restrict__ res_cols,
     const float* __restrict__ res_vals, const TB* __restrict__ B, int64_t ldb, uint32_t bbytes, int N,
-    float* __restrict__ C, int64_t ldc, int nC, int nC2, int nw, float* __restrict__ ws, int block0) {
+    float* __restrict__ C, int64_t ldc, int nC, int nC2, int nw, float* __restrict__ ws) {
   extern __shared__ float4 stream_lds[];
   float* lds = reinterpret_cast<float*>(stream_lds);
-  const StreamArrays A{p.tc_ptr, p.tc_cols, p.res_ptr, p.res_cols, p.win_rows, p.tc_vals, p.tc_scale, p.res_vals};
-  const int block = block0 + (int)blockIdx.x;
+  const int block = (int)blockIdx.x;
   const int big = (p.n_parts + p.W_big - p.W_huge) * nC2;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bool fold = p.fold_mix != 0;
@@ -345,12 +346,12 @@ __global__ __launch_bounds__(kStreamWaves * 64, 4) void hyb_spmm_stream_kernel(
     const int i = block / nC2, n0 = (block - i * nC2) * 32;
     if (i < p.n_parts) {
       const int w = p.part_win[i];
-      stream_window<MODE, TB, 2, kVec, kBuf>(A, res_ptr, res_cols, res_vals, B, ldb, bbytes, N, C, ldc, w, n0,
+      stream_window<MODE, TB, 2, kVec, kBuf>(p, res_ptr, res_cols, res_vals, B, ldb, bbytes, N, C, ldc, w, n0,
                                              p.part_c0[i], p.part_c1[i], i == p.hw_p0[w] && has_sparse(w),
                                              ws ? ws + (int64_t)i * 16 * N : nullptr, true, lds, wv, kStreamWaves);
     } else {
       const int w = p.W_huge + i - p.n_parts;
-      stream_window<MODE, TB, 2, kVec, kBuf>(A, res_ptr, res_cols, res_vals, B, ldb, bbytes, N, C, ldc, w, n0,
+      stream_window<MODE, TB, 2, kVec, kBuf>(p, res_ptr, res_cols, res_vals, B, ldb, bbytes, N, C, ldc, w, n0,
                                              p.tc_ptr[w], p.tc_ptr[w + 1], has_sparse(w), nullptr, false, lds, wv,
                                              kStreamWaves);
     }
@@ -365,7 +366,7 @@ __global__ __launch_bounds__(kStreamWaves * 64, 4) void hyb_spmm_stream_kernel(
   const bool live = p.W_big + i < p.W_tc;
   const int w = live ? p.W_big + i : p.W_tc - 1, n0 = live ? (job - i * nC) * 64 : N;
   const int c0 = p.tc_ptr[w], c1 = live ? p.tc_ptr[w + 1] : c0;
-  stream_window<MODE, TB, 4, kVec, kBuf>(A, res_ptr, res_cols, res_vals, B, ldb, bbytes, N, C, ldc, w, n0, c0, c1,
+  stream_window<MODE, TB, 4, kVec, kBuf>(p, res_ptr, res_cols, res_vals, B, ldb, bbytes, N, C, ldc, w, n0, c0, c1,
                                          live && has_sparse(w), nullptr, false, lds + sub * (nw + 1) * 16 * 64,
                                          wv - sub * nw, nw);
 }
@@ -402,10 +403,6 @@ template <typename TB>
 hipError_t launch_stream(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc, bool vec,
                          float* ws, hipStream_t s) {
   if (p.W_tc == 0) return hipSuccess;
-  if (p.n_parts > 0 && !ws) {
-    hipError_t e = launch_zero_window_rows(p, p.W_huge, C, ldc, N, s);
-    if (e != hipSuccess) return e;
-  }
   const int nC = (N + 63) / 64, nC2 = (N + 31) / 32;
   // Waves per (window, 64 columns): half a workgroup's when the windows hold few
   // chunks on average and there are enough of them to fill the GPU, else all.
@@ -414,16 +411,29 @@ hipError_t launch_stream(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, 
   const int nw = few && jobs >= 512 ? kStreamWaves / 2 : kStreamWaves;
   const int per = kStreamWaves / nw;
   const int64_t blocks = (int64_t)(p.n_parts + p.W_big - p.W_huge) * nC2 + (jobs + per - 1) / per;
-  if (blocks * per > INT32_MAX) return hipErrorInvalidValue;
+  if (blocks > max_blocks(kStreamWaves * 64) && N > 64) {
+    // in column halves: each a product of its own, with its part of ws (an offset
+    // of the blocks in the kernel would take scalar registers it does not have:
+    // 1024 x 4096, N = 512 14.9 -> 15.5 us)
+    const int n = nC / 2 * 64;
+    hipError_t e = launch_stream(p, B, ldb, n, C, ldc, vec, ws, s);
+    if (e != hipSuccess) return e;
+    return launch_stream(p, B + n, ldb, N - n, C + n, ldc, vec, ws ? ws + (int64_t)p.n_parts * 16 * n : nullptr, s);
+  }
+  if (p.n_parts > 0 && !ws) {
+    hipError_t e = launch_zero_window_rows(p, p.W_huge, C, ldc, N, s);
+    if (e != hipSuccess) return e;
+  }
   // 32-bit row offsets from 24-bit products
   uint32_t bytes = b_bytes<TB>(p.K, ldb, N);
   if (p.K > (1 << 24) || ldb * (int64_t)sizeof(TB) >= (1 << 24)) bytes = 0;
   const size_t lds = (size_t)(kStreamWaves + per) * 16 * 64 * 4;
-  int64_t b0 = 0, n = 0;
+  const StreamArrays arrays{p.tc_ptr,  p.tc_cols, p.win_rows, p.tc_vals, p.tc_scale, p.part_win, p.part_c0,
+                            p.part_c1, p.hw_p0,   p.W_tc,     p.W_big,   p.W_huge,   p.n_parts,  p.fold_mix};
   auto go = [&](auto mode, auto v, auto u) {
     hipLaunchKernelGGL((hyb_spmm_stream_kernel<decltype(mode)::value, TB, decltype(v)::value, decltype(u)::value>),
-                       dim3((unsigned)n), dim3(kStreamWaves * 64), lds, s, p, p.res_ptr, p.res_cols, p.res_vals, B,
-                       ldb, bytes, N, C, ldc, nC, nC2, nw, ws, (int)b0);
+                       dim3((unsigned)blocks), dim3(kStreamWaves * 64), lds, s, arrays, p.res_ptr, p.res_cols, p.res_vals, B,
+                       ldb, bytes, N, C, ldc, nC, nC2, nw, ws);
   };
   auto by_layout = [&](auto mode) {
     if (bytes > 0 && vec)
@@ -433,18 +443,14 @@ hipError_t launch_stream(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, 
     else
       go(mode, std::false_type{}, std::false_type{});
   };
-  hipError_t e = hipSuccess;
-  for (; b0 < blocks; b0 += n) {
-    n = std::min(blocks - b0, max_blocks(kStreamWaves * 64));
-    if (p.blk_dtype == 1)
-      by_layout(std::integral_constant<int, 1>{});
-    else if (p.blk_dtype == 2)
-      by_layout(std::integral_constant<int, 2>{});
-    else
-      by_layout(std::integral_constant<int, 0>{});
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
+  if (p.blk_dtype == 1)
+    by_layout(std::integral_constant<int, 1>{});
+  else if (p.blk_dtype == 2)
+    by_layout(std::integral_constant<int, 2>{});
+  else
+    by_layout(std::integral_constant<int, 0>{});
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
   if (ws && p.W_huge > 0) {
     const int64_t waves = (int64_t)p.W_huge * nC;
     hipLaunchKernelGGL(hyb_spmm_part_reduce_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, p, N, C, ldc,

@@ -3,7 +3,8 @@ fewer than 2^32 threads): few rows and 2^22 columns, so that the matrices stay s
 
 Every entry of C is written; columns at the ends, at the cuts and between are
 compared with FP64, per element within (n + 2) 2^-24 sum|a||b| for rows of n
-entries (n products, rounded and added in FP32 in some order)."""
+entries (n products, rounded and added in FP32 in some order), 2^-7 sum|a||b|
+for BF16 blocks (A rounded to BF16, 2^-9, the sums as above)."""
 import numpy as np
 import pytest
 import scipy.sparse
@@ -16,13 +17,13 @@ pytestmark = pytest.mark.gpu
 N = 1 << 22
 
 
-def _run(cuda, A, search, deterministic):
-    opts = api.options_for("float32")
+def _run(cuda, A, search, deterministic, blocks="float32", N=N):
+    opts = api.options_for(blocks)
     setattr(opts, search, True)
-    plan = _native.Plan.spmm(api.spmm_pack(A, opts)[0], "float32")
+    plan = _native.Plan.spmm(api.spmm_pack(A, opts)[0], blocks)
     g = torch.Generator(device=cuda)
     g.manual_seed(1)
-    B = torch.randn(A.shape[1], N, device=cuda, generator=g)
+    B = torch.randn(A.shape[1], N, device=cuda, generator=g, dtype=getattr(torch, blocks))
     C = torch.full((A.shape[0], N), float("nan"), device=cuda)
     print("launch limits", A.shape, A.nnz, search, deterministic, plan.info(), flush=True)
     plan.run_spmm(B, C, deterministic=deterministic)
@@ -31,7 +32,8 @@ def _run(cuda, A, search, deterministic):
     cols = torch.cat([torch.arange(130), torch.arange(N // 2 - 70, N // 2 + 70), torch.arange(N - 130, N),
                       torch.randint(N, (200,), generator=torch.Generator().manual_seed(2))]).to(cuda)
     A64, B64 = torch.from_numpy(A.toarray()).to(cuda).double(), B[:, cols].double()
-    bound = (np.diff(A.indptr).max() + 2) * 2.0 ** -24 * (A64.abs() @ B64.abs())
+    unit = (np.diff(A.indptr).max() + 2) * 2.0 ** -24 if blocks == "float32" else 2.0 ** -7
+    bound = unit * (A64.abs() @ B64.abs())
     assert torch.all((C[:, cols].double() - A64 @ B64).abs() <= bound)
     return plan.info()
 
@@ -64,3 +66,10 @@ def test_dense_windows(cuda):
     # 128 windows of 6 chunks, a workgroup for each 64 of 2^22 columns
     info = _run(cuda, _full(2048, 192), "only_TC", False)
     assert info["sparse_nnz"] == 0 and info["num_chunks"] == 768
+
+
+@pytest.mark.parametrize("deterministic", [False, True])
+def test_parts_of_huge_windows(cuda, deterministic):
+    # 64 windows of 257 chunks in two parts each, a workgroup for each 32 of 2^21 columns
+    info = _run(cuda, _full(1024, 8224), "only_TC", deterministic, "bfloat16", 1 << 21)
+    assert info["num_chunks"] == 64 * 257
