@@ -1,6 +1,8 @@
 // Fused sparse attention of libstile_hip.so for MI355X (gfx950).
 #include "stile_device.h"
 
+#include <algorithm>
+
 namespace stile {
 
 // ---------------------------------------------------------------------------
@@ -112,13 +114,20 @@ typedef int32_t i32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 // bank quadruples.
 constexpr int kAttOStride = 68;
 
+// What the kernel reads of a plan (a launch passes no more of it).
+struct AttArrays {
+  const int32_t *win_rows, *tc_ptr, *tc_cols;
+  const uint32_t* tc_mask;
+  const int32_t *res_ptr, *res_cols;
+};
+
 template <bool kSmall>
-__global__ __launch_bounds__(64, 3) void attention_fused_kernel(SpmmPlanDev p, AttOrder ord,
+__global__ __launch_bounds__(64, 3) void attention_fused_kernel(AttArrays p, AttOrder ord,
                                                                 const __bf16* __restrict__ Qm,
                                                                 const __bf16* __restrict__ Km,
                                                                 const __bf16* __restrict__ Vm, int64_t ld,
                                                                 float scale, float* __restrict__ out, int64_t ldo,
-                                                                int first) {
+                                                                uint32_t vbytes) {
   // the chunk's 32 K and 32 V rows; after them the sums on their way to the sparse part
   __shared__ __align__(16) unsigned char stage[64 * kAttVRow];
   static_assert(64 * kAttVRow >= 4 * 16 * kAttOStride);
@@ -131,7 +140,7 @@ __global__ __launch_bounds__(64, 3) void attention_fused_kernel(SpmmPlanDev p, A
       o0 = ord.start[i];
       o1 = ord.start[i + 1];
     }
-  const int oi = o0 + first + (int)(blockIdx.x / kXcds);
+  const int oi = o0 + (int)(blockIdx.x / kXcds);
   if (oi >= o1) return;
   const int w = __builtin_amdgcn_readfirstlane(ord.win[oi]);
   lds_u8* const vt = (lds_u8*)stage;
@@ -302,6 +311,7 @@ __global__ __launch_bounds__(64, 3) void attention_fused_kernel(SpmmPlanDev p, A
       const float4 v = ld4(os + sq * kAttOStride + 8 * s4 + (e < 8 ? e : 24 + e));
       om[e] = v.x; om[e + 1] = v.y; om[e + 2] = v.z; om[e + 3] = v.w;
     }
+    const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(Vm), 0, vbytes, 0x00020000);
     for (int j = 0; j < n; j += kAttBatch) {
       bf16x8 ka[kAttBatch], kb[kAttBatch], va[kAttBatch], vb[kAttBatch];
       bool on[kAttBatch];
@@ -311,8 +321,17 @@ __global__ __launch_bounds__(64, 3) void attention_fused_kernel(SpmmPlanDev p, A
         const Off off = row_off(on[u] ? sid[u] : 0, 16 * s4);
         ka[u] = row8(Km, off);
         kb[u] = row8(Km, off + 64);
-        va[u] = row8(Vm, off);
-        vb[u] = row8(Vm, off + 64);
+        // V of entries past a row's end is 0, whatever the rows hold (0 times an
+        // infinity or a NaN is a NaN): loads past the descriptor (64 masks of 640
+        // to 5,120 rows: 78.9 us a pass), or selects below (79.9)
+        if constexpr (kSmall) {
+          const uint32_t voff = on[u] ? off : vbytes;
+          va[u] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(vr, voff, 0, 0));
+          vb[u] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(vr, voff + 64, 0, 0));
+        } else {
+          va[u] = row8(Vm, off);
+          vb[u] = row8(Vm, off + 64);
+        }
       }
       load_cols(j + kAttBatch);
       __builtin_amdgcn_sched_barrier(0);  // every load of the step before its arithmetic
@@ -326,12 +345,12 @@ __global__ __launch_bounds__(64, 3) void attention_fused_kernel(SpmmPlanDev p, A
         sval[u] = on[u] ? dot : -INFINITY;
         m_run = fmaxf(m_run, sval[u]);
       }
-      // V rows read for entries past a row's end weigh nothing, whatever they hold
-      // (0 times an infinity or a NaN is a NaN)
-      if (!__all(on[kAttBatch - 1])) {
+      if constexpr (!kSmall) {
+        if (!__all(on[kAttBatch - 1])) {
 #pragma unroll
-        for (int u = 0; u < kAttBatch; ++u)
-          if (!on[u]) va[u] = vb[u] = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
+          for (int u = 0; u < kAttBatch; ++u)
+            if (!on[u]) va[u] = vb[u] = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
+        }
       }
       auto prob = [&](float x, float mx) { return x == -INFINITY ? 0.f : __expf((x - mx) * scale); };
       if (__all(m_run == ms)) {
@@ -387,19 +406,28 @@ hipError_t launch_attention(const SpmmPlanDev& p, const AttOrder& ord, const voi
   int longest = 0;
   for (int x = 0; x < kXcds; ++x) longest = max(longest, ord.start[x + 1] - ord.start[x]);
   // 32-bit row offsets from 24-bit products: up to 2^24 rows and 4 GiB (of Q: M,
-  // of K and V: K, equal in attention plans)
+  // of K and V: K, equal in attention plans), less a row so that offsets past V
+  // stay below 2^32
   const int64_t rows = max(p.M, p.K);
-  const bool small = rows < (1 << 24) && ld < (1 << 23) && rows * ld * 2 < ((int64_t)1 << 32);
+  const bool small = rows < (1 << 24) && ld < (1 << 23) && rows * ld * 2 < ((int64_t)1 << 32) - 256;
   const auto kernel = small ? attention_fused_kernel<true> : attention_fused_kernel<false>;
-  constexpr int kMost = (int)(max_blocks(64) / kXcds);
-  hipError_t e = hipSuccess;
-  for (int first = 0; first < longest && e == hipSuccess; first += kMost) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(min(kMost, longest - first) * kXcds)), dim3(64), 0, s, p, ord,
+  const AttArrays arrays{p.win_rows, p.tc_ptr, p.tc_cols, p.tc_mask, p.res_ptr, p.res_cols};
+  auto launch = [&](const AttOrder& o, int most) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(most * kXcds)), dim3(64), 0, s, arrays, o,
                        static_cast<const __bf16*>(Q), static_cast<const __bf16*>(K), static_cast<const __bf16*>(V),
-                       ld, scale, out, ldo, first);
-    e = hipGetLastError();
+                       ld, scale, out, ldo, small ? (uint32_t)((p.K - 1) * ld * 2 + 128) : 0u);
+    return hipGetLastError();
+  };
+  constexpr int kMost = (int)(max_blocks(64) / kXcds);  // windows per XCD of one launch
+  if (longest <= kMost) return launch(ord, longest);
+  AttOrder part = ord;  // in launches of equally many windows per XCD
+  for (int64_t a = 0; a < p.W; a = part.start[kXcds]) {
+    const int64_t n = std::min<int64_t>(p.W - a, (int64_t)kMost * kXcds);
+    for (int x = 0; x <= kXcds; ++x) part.start[x] = (int32_t)(a + n * x / kXcds);
+    const hipError_t e = launch(part, (int)((n + kXcds - 1) / kXcds));
+    if (e != hipSuccess) return e;
   }
-  return e;
+  return hipSuccess;
 }
 
 }  // namespace stile
