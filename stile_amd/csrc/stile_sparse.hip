@@ -199,25 +199,22 @@ int row_width(int N, int K, int elem, int64_t waves) {
   return wide && N > 64 && waves * chunks >= kFewWaves ? 2 : 1;
 }
 
-// f(VW, kVec, kBuf) with all three as compile-time constants.
+// f(VW, kVec, kBuf) with all three as compile-time constants.  One column per
+// lane is the same code aligned or not.
 template <typename F>
 void with_width(int vw, bool vec, bool buf, F&& f) {
-  auto g = [&](auto w) {
-    auto h = [&](auto v) {
-      if (buf)
-        f(w, v, std::true_type{});
-      else
-        f(w, v, std::false_type{});
-    };
-    if (vec)
-      h(std::true_type{});
+  auto g = [&](auto w, auto v) {
+    if (buf)
+      f(w, v, std::true_type{});
     else
-      h(std::false_type{});
+      f(w, v, std::false_type{});
   };
-  if (vw == 2)
-    g(std::integral_constant<int, 2>{});
+  if (vw == 1)
+    g(std::integral_constant<int, 1>{}, std::false_type{});
+  else if (vec)
+    g(std::integral_constant<int, 2>{}, std::true_type{});
   else
-    g(std::integral_constant<int, 1>{});
+    g(std::integral_constant<int, 2>{}, std::false_type{});
 }
 
 }  // namespace
