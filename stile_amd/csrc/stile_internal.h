@@ -29,18 +29,27 @@ constexpr int32_t kTaskSlots = 0x3fffffff, kTaskAdd = 0x40000000, kTaskHub = (in
 // Value id of an A element that a value refresh leaves as it is (the row
 // half of a scatter chunk's k-slot word).
 constexpr int32_t kKeepId = -2;
-// The streaming kernel gives each (window, 64 columns) a workgroup, each of its
-// waves a contiguous share of the window's chunks, and sums the partial results
-// through LDS in wave order.  Windows with more than kBigChunks chunks are "big"
-// and take 32 columns a workgroup: twice the workgroups, and four chunks in
-// flight per wave instead of two, for the windows a launch waits for.
+// The streaming kernel (launches that leave the GPU partly idle, full_launch) gives
+// each (window, 64 columns) a workgroup or half of one, each of its waves a
+// contiguous share of the window's chunks, and sums the partial results through LDS
+// in wave order.  Windows with more than kBigChunks chunks are "big" and take 32
+// columns a workgroup: twice the workgroups, and four chunks in flight per wave
+// instead of two, for the windows a launch waits for.  64 FP32 windows of 24 chunks,
+// N = 128: 6.6 us, 9.9 on 64 columns; the line at 12 chunks instead of 16 made a 4096
+// x 4096 FP32 layer at N = 256 slower, 31.9 -> 38.6 us.
 constexpr int kBigChunks = 16;
-// Windows with more than kLongChunks chunks come first in a plan, most chunks first.
+// Windows with more than kLongChunks chunks come first in a plan, most chunks first
+// (512 windows of 2, 9 and one of 47 chunks, N = 256: 13.6 us; with only those of more
+// than 16 in front 16.0), and share a workgroup in full launches.
 constexpr int kLongChunks = 8;
-// Sparse parts of dense windows whose rows have at most this many entries are
+constexpr int kStreamWaves = 8;  // waves of a streaming workgroup
+// Sparse parts of dense windows whose rows have at most this many entries may be
 // summed by the streaming kernel's workgroup of the window (no second launch, no
-// second pass over C); longer ones by the sparse-row kernel's tasks, which are
-// balanced over the whole GPU.
+// second pass over C; kFoldWave), longer ones are left to the sparse-row kernel's
+// tasks, which are balanced over the whole GPU.  64 BF16 windows of 100 columns, N =
+// 512, one row of 16 with 128 entries: 8.9 us, 13.5 by tasks; with 256 12.8 and 19.3,
+// so the line is not where folding stops to pay but leaves no row of kSplitNnz entries
+// and more, whose rest is in pieces.
 constexpr int kFoldMaxLen = 128;
 // Windows with more than kHugeChunks chunks (hub rows of power-law graphs)
 // are cut into parts of at most kHugeChunks chunks, one workgroup each, that
@@ -90,9 +99,12 @@ struct LdsXcdRanges {
 struct SpmmPlanDev {
   int32_t M, K, W;
   int32_t W_tc;              // windows [0, W_tc) hold dense chunks; the rest are sparse-only
+  int32_t W_long;            // windows [0, W_long) hold more than kLongChunks chunks (0: B-stationary plans)
   int32_t W_big;             // windows [0, W_big) hold more than kBigChunks chunks
   int32_t W_huge;            // windows [0, W_huge) hold more than kHugeChunks chunks
   int32_t chunks_small;      // chunks of windows [W_big, W_tc)
+  int32_t full_chain;        // most chunks a wave of a full launch runs in sequence (full_launch)
+  int32_t nnz_mix;           // sparse nonzeros in windows [0, W_tc)
   int32_t n_parts;           // parts of the huge windows
   const int32_t* part_win;   // [n_parts] window of each part
   const int32_t* part_c0;    // [n_parts] chunk range of each part
@@ -153,7 +165,7 @@ struct SpmmPlanDev {
   int32_t n_row_tasks, n_mix_tasks;
   const int2* row_tasks;
   int32_t n_mix;             // slots of dense windows with a sparse part
-  int32_t fold_mix;          // 1: none of them holds more than kFoldMaxLen entries
+  int32_t fold_mix;          // 1: the streaming kernel may sum them (kFoldMaxLen, kFoldWindow)
   const uint32_t* tc_mask;   // [nchunks][16] entry bits (attention plans), else nullptr
   // B-stationary work units (BF16 plans with every matrix's K <= kLdsMaxK):
   // unit = (first window, end window, first B row, B rows) of one matrix,
@@ -254,12 +266,12 @@ hipError_t launch_zero_window_rows(const SpmmPlanDev& p, int nwin, float* C, int
 hipError_t launch_row_softmax(int M, const int32_t* indptr, const float* in, float* out, float scale,
                               hipStream_t s);
 
-// Dense windows on the streaming kernel (with their sparse parts when the plan
-// folds them, SpmmPlanDev::fold_mix).  ws: the deterministic mode's region for
-// the parts of huge windows, nullptr to add them with atomicAdd.
+// Dense windows on the streaming kernels.  *folded: their sparse parts are in C
+// (else the sparse-row tasks are to add them).  ws: the deterministic mode's
+// region for the parts of huge windows, nullptr to add them with atomicAdd.
 template <typename TB>
 hipError_t launch_stream(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc, bool vec,
-                         float* ws, hipStream_t s);
+                         float* ws, hipStream_t s, bool* folded);
 
 // out (F x Fg) = H^T G over M rows; ws: slabs * F * Fg floats (tall_slabs gives
 // the slab count and rows per slab).  H and G each span less than 4 GiB.

@@ -960,9 +960,10 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
   const int cus = device_cus();
   const bool fold = lds && so_rows > 0 && so_rows * nC <= kLdsTailMaxTasks &&
                     (so_rows * nC + kLdsThreads / 64 - 1) / (kLdsThreads / 64) <= cus / kXcds * kXcds;
-  // The LDS kernel runs every dense window with its sparse part; otherwise
-  // the streaming kernel does the dense parts (its first blocks the big
-  // windows) and the sparse kernel the sparse parts.
+  // The LDS kernel runs every dense window with its sparse part; otherwise a
+  // streaming kernel does the dense parts and, when the sparse parts are short
+  // and the launch small, those too (folded); else the row tasks add them.
+  bool folded = true;
   if (lds) {
     int t = p.opt_lds_list >= 0 && p.opt_lds_list < kLdsLists ? p.opt_lds_list : -1;
     if (t < 0 && nC <= kLdsPickMax) t = p.lds_pick[nC];
@@ -1021,7 +1022,7 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   } else if (p.W_tc > 0) {
-    hipError_t e = launch_stream(p, B, ldb, N, C, ldc, vec, ws_parts, s);
+    hipError_t e = launch_stream(p, B, ldb, N, C, ldc, vec, ws_parts, s, &folded);
     if (e != hipSuccess) return e;
   }
   // Sparse-only rows (unless they were the LDS launch's tail) by wave tasks, or,
@@ -1039,7 +1040,7 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
     if (e != hipSuccess) return e;
   }
   {
-    hipError_t e = launch_sparse_rows(p, B, ldb, N, C, ldc, vec, lds ? p.n_mix_tasks : 0,
+    hipError_t e = launch_sparse_rows(p, B, ldb, N, C, ldc, vec, folded ? p.n_mix_tasks : 0,
                                       so_left > 0 && !split ? p.n_row_tasks : p.n_mix_tasks, s);
     if (e != hipSuccess) return e;
   }

@@ -755,7 +755,7 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   // by matrix (and no window counts as big or huge, which only the streaming
   // kernel uses).
   const bool by_matrix = lds_ok && bd.inst_rows.size() > 2;
-  int32_t W_big = 0, W_huge = 0;
+  int32_t W_long = 0, W_big = 0, W_huge = 0;
   if (by_matrix) {
     std::vector<int32_t> mat(W);
     for (int32_t w = 0; w < W; ++w) mat[w] = window_matrix(bd, w);
@@ -764,6 +764,7 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
     auto long_end = std::stable_partition(order.begin(), order.begin() + W_tc,
                                           [&](int32_t w) { return nch(w) > stile::kLongChunks; });
     std::stable_sort(order.begin(), long_end, [&](int32_t a, int32_t b) { return nch(a) > nch(b); });
+    W_long = (int32_t)(long_end - order.begin());
     while (W_big < W_tc && nch(order[W_big]) > stile::kBigChunks) ++W_big;
     while (W_huge < W_big && nch(order[W_huge]) > stile::kHugeChunks) ++W_huge;
   }
@@ -819,8 +820,8 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
     }
   }
   // Slots of dense windows that also have a sparse part: summed with the window
-  // when they are short (fold_mix), else added to the rows the streaming kernel
-  // stored by the sparse rows' tasks.
+  // when they are short (fold_mix) and the launch small, else added to the rows the
+  // streaming kernel stored by the sparse rows' tasks.
   int32_t n_mix = 0;
   int64_t longest_mix = 0;
   for (int64_t sl = 0; sl < (int64_t)W_tc * 16; ++sl)
@@ -856,7 +857,7 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   }
 
   std::vector<int32_t> row_tasks;
-  if (!fold_mix) sparse_row_tasks(cnt, 0, (int64_t)W_tc * 16, stile::kTaskAdd, row_tasks);
+  sparse_row_tasks(cnt, 0, (int64_t)W_tc * 16, stile::kTaskAdd, row_tasks);
   const int32_t n_mix_tasks = (int32_t)(row_tasks.size() / 2);
   sparse_row_tasks(cnt, (int64_t)W_tc * 16, (int64_t)W * 16, 0, row_tasks);
 
@@ -1131,9 +1132,16 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   d.K = bd.K;
   d.W = W;
   d.W_tc = W_tc;
+  d.W_long = W_long;
   d.W_big = W_big;
   d.W_huge = W_huge;
   d.chunks_small = tc_ptr[W_tc] - tc_ptr[W_big];
+  d.full_chain = 0;
+  for (int32_t w = 0; w < W_tc; ++w) {
+    const int32_t n = std::min(tc_ptr[w + 1] - tc_ptr[w], stile::kHugeChunks);
+    d.full_chain = std::max(d.full_chain, w < W_long ? (n + stile::kStreamWaves - 1) / stile::kStreamWaves : n);
+  }
+  d.nnz_mix = res_ptr[(size_t)W_tc * 16];
   d.n_parts = (int32_t)part_win.size();
   d.part_win = dptr<int32_t>(plan, o_pwin);
   d.part_c0 = dptr<int32_t>(plan, o_pc0);

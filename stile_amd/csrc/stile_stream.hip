@@ -7,10 +7,11 @@
 namespace stile {
 
 // ---------------------------------------------------------------------------
-// One workgroup = (window or part of a huge window, 16 * NT columns).  Each wave
-// takes a contiguous share of the window's chunks and, in plans that fold the
-// sparse parts, some of its 16 slots' sparse entries; the partial sums meet in
-// LDS, are added in wave order and leave as whole rows of C.
+// hyb_spmm_stream_kernel: one workgroup, or half of one, = (window or part of a
+// huge window, 16 * NT columns).  Each wave takes a contiguous share of the window's
+// chunks and, in launches that fold the sparse parts, some of its 16 slots' sparse
+// entries; the partial sums meet in LDS, are added in wave order and leave as whole
+// rows of C.
 //
 // Lane l = 16g + j of a wave holds, for MFMA tile t, column col(j, t) of rows 4g
 // .. 4g + 3 of the window: kVec (B rows aligned, N % 4 == 0) n0 + NT j + t, so
@@ -33,10 +34,11 @@ namespace stile {
 // in sequence, and a 1024 x 4096 BF16 layer (N = 512) took 24 us.  With four to
 // eight waves per window, up to four chunks in flight, 32 columns a workgroup
 // for windows of more than 16 chunks and the sparse parts in the same launch:
-// 8.7, 38 and 14.9 us.
+// 8.7, 38 and 14.9 us.  Launches that fill the GPU without all that have a kernel of
+// their own (hyb_spmm_stream_full_kernel, full_launch): the 3072 x 768 FP16 layer at
+// N = 4096 takes 33 us on it, 64 on several waves a window and 42 on the one-wave
+// kernel before either; in FP32 65, 81 and 78.
 // ---------------------------------------------------------------------------
-constexpr int kStreamWaves = 8;
-
 // B elements of one chunk's eight rows for this lane, as loaded.
 template <typename TB, int NT, bool kVec>
 struct ChunkB {
@@ -186,7 +188,7 @@ struct StreamArrays {
   const void* tc_vals;
   const float* tc_scale;
   const int32_t *part_win, *part_c0, *part_c1, *hw_p0;
-  int32_t W_tc, W_big, W_huge, n_parts, fold_mix;
+  int32_t W_tc, W_long, W_big, W_huge, n_parts, fold_mix;
 };
 
 // Registers for the chunks in flight (four waves per SIMD).  16-bit rows with
@@ -209,7 +211,7 @@ __device__ __forceinline__ void stream_window(const StreamArrays& A, const int32
   static_assert(D >= 1);
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, j = lane & 15;
-  const int share = max((c1 - c0 + nw - 1) / nw, 1);  // (no chunks: see the kernel's last job)
+  const int share = (c1 - c0 + nw - 1) / nw;
   const int nd = (c1 - c0 + share - 1) / share;  // waves with a share
   const int a = min(c0 + wv * share, c1), b = min(a + share, c1);
   // Sparse entries of the window's slots: on the waves without chunks when they
@@ -357,18 +359,119 @@ __global__ __launch_bounds__(kStreamWaves * 64, 4) void hyb_spmm_stream_kernel(
     }
     return;
   }
-  // kStreamWaves / nw windows side by side; a last workgroup with fewer left runs
-  // the spare waves on no chunks and columns from N on, so that every wave meets
-  // the others at the same barrier and stores nothing
+  // kStreamWaves / nw windows side by side.  Waves of a last workgroup that have no
+  // window left end here: the barrier waits for the waves that have not ended.
   const int sub = wv / nw;
   const int job = (block - big) * (kStreamWaves / nw) + sub;
-  const int i = job / nC;
-  const bool live = p.W_big + i < p.W_tc;
-  const int w = live ? p.W_big + i : p.W_tc - 1, n0 = live ? (job - i * nC) * 64 : N;
-  const int c0 = p.tc_ptr[w], c1 = live ? p.tc_ptr[w + 1] : c0;
-  stream_window<MODE, TB, 4, kVec, kBuf>(p, res_ptr, res_cols, res_vals, B, ldb, bbytes, N, C, ldc, w, n0, c0, c1,
-                                         live && has_sparse(w), nullptr, false, lds + sub * (nw + 1) * 16 * 64,
-                                         wv - sub * nw, nw);
+  const int i = job / nC, n0 = (job - i * nC) * 64;
+  const int w = p.W_big + i;
+  if (w >= p.W_tc) return;
+  stream_window<MODE, TB, 4, kVec, kBuf>(p, res_ptr, res_cols, res_vals, B, ldb, bbytes, N, C, ldc, w, n0,
+                                         p.tc_ptr[w], p.tc_ptr[w + 1], has_sparse(w), nullptr, false,
+                                         lds + sub * (nw + 1) * 16 * 64, wv - sub * nw, nw);
+}
+
+// Chunks [a, b) of a window into acc, two at a time, the column ids of the next
+// two requested under the current ones' B rows.
+template <int MODE, typename TB, bool kVec, bool kBuf>
+__device__ __forceinline__ void full_chunks(const StreamArrays& A, const ChunkReader<TB, 4, kVec, kBuf>& rd, int a,
+                                            int b, f32x4 (&acc)[4]) {
+  const int g = (threadIdx.x & 63) >> 4;
+  struct Ids {
+    int4 ka, kb;
+  };
+  auto ids_of = [&](int c) {
+    const int4* cp = reinterpret_cast<const int4*>(A.tc_cols + (int64_t)min(c, b - 1) * 32 + g * 8);
+    return Ids{cp[0], cp[1]};
+  };
+  Ids i0 = ids_of(a), i1 = ids_of(a + 1);
+  int c = a;
+  for (; c + 1 < b; c += 2) {
+    ChunkA<MODE> a0, a1;
+    ChunkB<TB, 4, kVec> b0, b1;
+    a0.load(A.tc_vals, A.tc_scale, c);
+    a1.load(A.tc_vals, A.tc_scale, c + 1);
+    rd.load(i0.ka, i0.kb, b0);
+    rd.load(i1.ka, i1.kb, b1);
+    i0 = ids_of(c + 2);
+    i1 = ids_of(c + 3);
+    mfma_chunk<MODE>(a0, b0, acc);
+    mfma_chunk<MODE>(a1, b1, acc);
+  }
+  if (c < b) {
+    ChunkA<MODE> a0;
+    ChunkB<TB, 4, kVec> b0;
+    a0.load(A.tc_vals, A.tc_scale, c);
+    rd.load(i0.ka, i0.kb, b0);
+    mfma_chunk<MODE>(a0, b0, acc);
+  }
+}
+
+// Launches that fill the GPU with a wave per (window, 64 columns) (full_launch):
+// blocks [0, (n_parts + W_long - W_huge) * nC) each run one (part, or window of
+// more than kLongChunks chunks) on all their waves, a contiguous share each, whose
+// sums the first wave adds in wave order; the next ones run kStreamWaves of the
+// other (window, 64 columns), one per wave, stored from its registers.
+template <int MODE, typename TB, bool kVec, bool kBuf>
+__global__ __launch_bounds__(kStreamWaves * 64) void hyb_spmm_stream_full_kernel(
+    StreamArrays p, const TB* __restrict__ B, int64_t ldb, uint32_t bbytes, int N, float* __restrict__ C, int64_t ldc,
+    int nC, float* __restrict__ ws) {
+  __shared__ f32x4 sums[kStreamWaves - 1][4][64];
+  const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int shared = (p.n_parts + p.W_long - p.W_huge) * nC;
+  const bool alone = (int)blockIdx.x >= shared;
+  const int job = alone ? ((int)blockIdx.x - shared) * kStreamWaves + wv : (int)blockIdx.x;
+  const int i = job / nC, n0 = (job - i * nC) * 64;
+  const bool in_part = !alone && i < p.n_parts;
+  const int w = alone ? p.W_long + i : in_part ? p.part_win[i] : p.W_huge + i - p.n_parts;
+  if (alone && w >= p.W_tc) return;
+  const int c0 = in_part ? p.part_c0[i] : p.tc_ptr[w], c1 = in_part ? p.part_c1[i] : p.tc_ptr[w + 1];
+  const int share = (c1 - c0 + kStreamWaves - 1) / kStreamWaves;
+  const int a = alone ? c0 : min(c0 + wv * share, c1), b = alone ? c1 : min(a + share, c1);
+  // rows before any store: vector-memory counters complete in issue order
+  int row[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) row[r] = p.win_rows[w * 16 + 4 * g + r];
+  f32x4 acc[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (a < b) full_chunks<MODE>(p, ChunkReader<TB, 4, kVec, kBuf>(B, ldb, bbytes, n0, N), a, b, acc);
+  if (!alone) {  // the whole workgroup
+    if (wv > 0) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) sums[wv - 1][t][lane] = acc[t];
+    }
+    __syncthreads();
+    if (wv > 0) return;
+    for (int v = 0; v < kStreamWaves - 1; ++v)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[t] += sums[v][t][lane];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float* at = in_part && ws ? ws + ((int64_t)i * 16 + 4 * g + r) * N : C + (int64_t)row[r] * ldc;
+    const bool out = (in_part && ws) || row[r] >= 0;
+    auto col = [&](int t) { return n0 + (kVec ? 4 * j + t : 16 * t + j); };
+    if (in_part && !ws) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (out && col(t) < N) atomicAdd(at + col(t), acc[t][r]);
+    } else if constexpr (kVec) {
+      if (out && col(0) < N) {
+        if (in_part) {  // rows of ws are aligned for a float only
+#pragma unroll
+          for (int t = 0; t < 4; ++t) at[col(t)] = acc[t][r];
+        } else {
+          st4(at + col(0), make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]));
+        }
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (out && col(t) < N) at[col(t)] = acc[t][r];
+    }
+  }
 }
 
 // Deterministic mode: C rows of huge window w = sum of its parts' partial
@@ -399,26 +502,72 @@ __global__ __launch_bounds__(256) void hyb_spmm_part_reduce_kernel(SpmmPlanDev p
   }
 }
 
+// Waves per (window, 64 columns) of hyb_spmm_stream_kernel: half a workgroup's
+// when the windows hold few chunks on average and there are enough of them to fill
+// the GPU, else all.  Windows of four chunks, FP32, four waves / eight: 512
+// (window, 64 columns) 6.0 / 6.0 us, 1,024 7.3 / 8.3; of eight chunks 7.1 / 6.3
+// and 12.3 / 10.5.
+static int waves_per_window(const SpmmPlanDev& p, int nC) {
+  const int64_t small = p.W_tc - p.W_big;
+  return small > 0 && p.chunks_small <= 4 * small && small * nC >= 512 ? kStreamWaves / 2 : kStreamWaves;
+}
+
+// Whether hyb_spmm_stream_full_kernel runs the dense windows.  Several waves per
+// window and their sum through LDS are for launches that leave the GPU idle; with
+// two waves per SIMD and more of one-wave (window, 64 columns) they only cost.
+// Windows of one chunk, full / not: FP32, 1,024 of them 5.3 / 5.3 us, 2,048 5.3 /
+// 8.3, 8,192 12.6 / 29.0; of eight chunks 15.5 / 12.3, 17.7 / 22.0 and 47 / 73;
+// BF16 of eight chunks 8.4 / 7.6, 9.3 / 12.9 and 25.9 / 49.  A window that a whole
+// workgroup shares counts as its eight waves where there are no others (17 chunks,
+// FP32, 128 / 256 of them: 6.3 / 5.9 and 6.5 / 9.4), as one beside windows of up to
+// eight chunks in one wave (2048 x 1024 FP16 layer, N = 512 9.4 / 8.1, N = 1024
+// 10.5 / 13.3).  Up to two chunks in sequence it is never behind.
+//
+// With sparse parts in the windows a full launch leaves them to the row tasks: a
+// launch (4 us) and a second pass over their rows of C (0.11 ns per row and 64
+// columns), against 2.5 ns per (window, 64 columns) beyond 1,024.  3072 x 768 FP32
+// layer, full / not: N = 1024 28.1 / 26.2 us, N = 2048 40.8 / 45.4, N = 4096 65 / 81.
+// Not with windows of more than kLongChunks chunks beside them (graphs; R-MAT scale
+// 15, N = 256: 97.6 / 86.9).
+static bool full_launch(const SpmmPlanDev& p, int nC) {
+  const int64_t alone = (int64_t)(p.W_tc - p.W_long) * nC;
+  const int64_t shared = (int64_t)(p.n_parts + p.W_long - p.W_huge) * nC;
+  if (p.nnz_mix == 0) return p.full_chain <= 2 || alone + shared * (alone == 0 ? kStreamWaves : 1) >= 1536;
+  return p.W_long == 0 && 250 * (alone - 1024) >= 400000 + 11 * (int64_t)p.n_mix * nC;
+}
+
+// Whether the windows' sparse parts are summed by hyb_spmm_stream_kernel: up to
+// kFoldWave entries per wave of a window on average, or kFoldTotal (entry, 64
+// columns) in all.  Above, the row tasks' gathers of 128 columns and their balance
+// are worth the second launch.  Folded / not: 64 BF16 windows of 100 columns, N =
+// 512 (four waves), 128 entries a wave and 262,144 in all 9.2 / 10.4 us, twice as
+// many 14.1 / 12.6; 512 of 40 columns, N = 128 (four waves), 32 a wave 8.6 / 10.7,
+// 128 and 524,288 17.8 / 14.1, 512 54 / 27; 4096 x 4096 layer, FP32, N = 256 (eight
+// waves, 73 a wave) 31.9 / 36.2.  One row of 16 with kFoldMaxLen entries, four in
+// the others: 8.9 / 13.5.
+constexpr int64_t kFoldWave = 96, kFoldTotal = 300000;
+
+// The launch over columns [0, N) of B and C; ws as in launch_stream.
 template <typename TB>
-hipError_t launch_stream(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc, bool vec,
-                         float* ws, hipStream_t s) {
-  if (p.W_tc == 0) return hipSuccess;
+static hipError_t stream_columns(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc,
+                                 bool vec, float* ws, hipStream_t s, bool full, int fold) {
   const int nC = (N + 63) / 64, nC2 = (N + 31) / 32;
-  // Waves per (window, 64 columns): half a workgroup's when the windows hold few
-  // chunks on average and there are enough of them to fill the GPU, else all.
   const int64_t jobs = (int64_t)(p.W_tc - p.W_big) * nC;
-  const bool few = p.W_tc > p.W_big && p.chunks_small <= (int64_t)4 * (p.W_tc - p.W_big);
-  const int nw = few && jobs >= 512 ? kStreamWaves / 2 : kStreamWaves;
+  const int nw = waves_per_window(p, nC);
   const int per = kStreamWaves / nw;
-  const int64_t blocks = (int64_t)(p.n_parts + p.W_big - p.W_huge) * nC2 + (jobs + per - 1) / per;
+  const int64_t blocks =
+      full ? (int64_t)(p.n_parts + p.W_long - p.W_huge) * nC +
+                 ((int64_t)(p.W_tc - p.W_long) * nC + kStreamWaves - 1) / kStreamWaves
+           : (int64_t)(p.n_parts + p.W_big - p.W_huge) * nC2 + (jobs + per - 1) / per;
   if (blocks > max_blocks(kStreamWaves * 64) && N > 64) {
     // in column halves: each a product of its own, with its part of ws (an offset
     // of the blocks in the kernel would take scalar registers it does not have:
     // 1024 x 4096, N = 512 14.9 -> 15.5 us)
     const int n = nC / 2 * 64;
-    hipError_t e = launch_stream(p, B, ldb, n, C, ldc, vec, ws, s);
+    const hipError_t e = stream_columns(p, B, ldb, n, C, ldc, vec, ws, s, full, fold);
     if (e != hipSuccess) return e;
-    return launch_stream(p, B + n, ldb, N - n, C + n, ldc, vec, ws ? ws + (int64_t)p.n_parts * 16 * n : nullptr, s);
+    return stream_columns(p, B + n, ldb, N - n, C + n, ldc, vec, ws ? ws + (int64_t)p.n_parts * 16 * n : nullptr, s,
+                          full, fold);
   }
   if (p.n_parts > 0 && !ws) {
     hipError_t e = launch_zero_window_rows(p, p.W_huge, C, ldc, N, s);
@@ -428,12 +577,17 @@ hipError_t launch_stream(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, 
   uint32_t bytes = b_bytes<TB>(p.K, ldb, N);
   if (p.K > (1 << 24) || ldb * (int64_t)sizeof(TB) >= (1 << 24)) bytes = 0;
   const size_t lds = (size_t)(kStreamWaves + per) * 16 * 64 * 4;
-  const StreamArrays arrays{p.tc_ptr,  p.tc_cols, p.win_rows, p.tc_vals, p.tc_scale, p.part_win, p.part_c0,
-                            p.part_c1, p.hw_p0,   p.W_tc,     p.W_big,   p.W_huge,   p.n_parts,  p.fold_mix};
+  const StreamArrays arrays{p.tc_ptr,  p.tc_cols, p.win_rows, p.tc_vals, p.tc_scale, p.part_win, p.part_c0, p.part_c1,
+                            p.hw_p0,   p.W_tc,    p.W_long,   p.W_big,   p.W_huge,   p.n_parts,  fold};
   auto go = [&](auto mode, auto v, auto u) {
-    hipLaunchKernelGGL((hyb_spmm_stream_kernel<decltype(mode)::value, TB, decltype(v)::value, decltype(u)::value>),
-                       dim3((unsigned)blocks), dim3(kStreamWaves * 64), lds, s, arrays, p.res_ptr, p.res_cols, p.res_vals, B,
-                       ldb, bytes, N, C, ldc, nC, nC2, nw, ws);
+    constexpr int kMode = decltype(mode)::value;
+    constexpr bool kV = decltype(v)::value, kU = decltype(u)::value;
+    if (full)
+      hipLaunchKernelGGL((hyb_spmm_stream_full_kernel<kMode, TB, kV, kU>), dim3((unsigned)blocks),
+                         dim3(kStreamWaves * 64), 0, s, arrays, B, ldb, bytes, N, C, ldc, nC, ws);
+    else
+      hipLaunchKernelGGL((hyb_spmm_stream_kernel<kMode, TB, kV, kU>), dim3((unsigned)blocks), dim3(kStreamWaves * 64),
+                         lds, s, arrays, p.res_ptr, p.res_cols, p.res_vals, B, ldb, bytes, N, C, ldc, nC, nC2, nw, ws);
   };
   auto by_layout = [&](auto mode) {
     if (bytes > 0 && vec)
@@ -460,11 +614,21 @@ hipError_t launch_stream(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, 
   return e;
 }
 
+template <typename TB>
+hipError_t launch_stream(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc, bool vec,
+                         float* ws, hipStream_t s, bool* folded) {
+  const int nC = (N + 63) / 64;
+  const bool full = full_launch(p, nC);
+  *folded = p.fold_mix && !full &&
+            (p.nnz_mix <= kFoldWave * waves_per_window(p, nC) * p.W_tc || (int64_t)p.nnz_mix * nC <= kFoldTotal);
+  return p.W_tc > 0 ? stream_columns(p, B, ldb, N, C, ldc, vec, ws, s, full, *folded) : hipSuccess;
+}
+
 template hipError_t launch_stream<float>(const SpmmPlanDev&, const float*, int64_t, int, float*, int64_t, bool, float*,
-                                         hipStream_t);
+                                         hipStream_t, bool*);
 template hipError_t launch_stream<__bf16>(const SpmmPlanDev&, const __bf16*, int64_t, int, float*, int64_t, bool,
-                                          float*, hipStream_t);
+                                          float*, hipStream_t, bool*);
 template hipError_t launch_stream<_Float16>(const SpmmPlanDev&, const _Float16*, int64_t, int, float*, int64_t, bool,
-                                            float*, hipStream_t);
+                                            float*, hipStream_t, bool*);
 
 }  // namespace stile
