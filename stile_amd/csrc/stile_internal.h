@@ -19,6 +19,9 @@ constexpr int kHubNnz = 4096;
 // mode: stores to a workspace, summed in piece order by a reduce kernel).
 constexpr int kSplitNnz = 256;
 
+// Sparse-only rows that are even (see even_rows_fit).
+constexpr int kEvenPercent = 135, kEvenMean = 16;
+
 // Entries of padding (column 0, value 0) behind res_cols and res_vals, for
 // kernels that read a row's entries a few at a time.
 constexpr int kRowPad = 32;
@@ -159,6 +162,7 @@ struct SpmmPlanDev {
   const int32_t* res_cols;
   const float* res_vals;
   int32_t nnz_sparse_only;   // sparse nonzeros in windows [W_tc, W)
+  int32_t even_rows;         // 1: their rows are even
   // wave tasks of hyb_spmm_rows_kernel: consecutive slots [x, y & kTaskSlots)
   // with the flags kTaskHub and kTaskAdd in y; the first n_mix_tasks are slots
   // of dense windows, the others of sparse-only windows
@@ -241,6 +245,10 @@ int64_t spmm_workspace_floats(const SpmmPlanDev& p, int N);
 template <typename TB>
 hipError_t launch_sparse_rows(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc, bool vec,
                               int t0, int t1, hipStream_t s);
+// The sparse-only windows by hyb_spmm_even_rows_kernel, where even_rows_fit.
+bool even_rows_fit(const SpmmPlanDev& p, int N, bool vec);
+hipError_t launch_even_rows(const SpmmPlanDev& p, const float* B, int64_t ldb, int N, float* C, int64_t ldc,
+                            hipStream_t s);
 template <typename TB>
 hipError_t launch_sparse_pieces(const SpmmPlanDev& p, const TB* B, int64_t ldb, int N, float* C, int64_t ldc,
                                 bool vec, int pc0, int pc1, float* ws, hipStream_t s);

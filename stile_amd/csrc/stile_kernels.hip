@@ -1027,9 +1027,9 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
   }
   // Sparse-only rows (unless they were the LDS launch's tail) by wave tasks, or,
   // when there are fewer than 16,384 (row, 64 columns) of 8 or more nonzeros on
-  // average, one of those per wave with all its gathers in flight at once.  The
-  // sparse parts of dense windows come first in the task list, when neither the
-  // LDS nor the streaming kernel added them.
+  // average, one of those per wave with all its gathers in flight at once, or one
+  // row per lane group when they are even.  The sparse parts of dense windows come
+  // first in the task list, when neither the LDS nor the streaming kernel added them.
   const int64_t so_left = fold ? 0 : so_rows;
   const bool split = so_left > 0 && so_left * nC / 4 < 4096 && p.nnz_sparse_only >= 8 * so_left;
   if (split) {
@@ -1039,9 +1039,17 @@ static hipError_t launch_hyb_spmm_t(const SpmmPlanDev& p, const TB* B, int64_t l
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
+  bool even = false;
+  if constexpr (std::is_same<TB, float>::value) {
+    even = so_left > 0 && !split && even_rows_fit(p, N, vec);
+    if (even) {
+      hipError_t e = launch_even_rows(p, B, ldb, N, C, ldc, s);
+      if (e != hipSuccess) return e;
+    }
+  }
   {
     hipError_t e = launch_sparse_rows(p, B, ldb, N, C, ldc, vec, folded ? p.n_mix_tasks : 0,
-                                      so_left > 0 && !split ? p.n_row_tasks : p.n_mix_tasks, s);
+                                      so_left > 0 && !split && !even ? p.n_row_tasks : p.n_mix_tasks, s);
     if (e != hipSuccess) return e;
   }
   // Pieces of long rows.  The LDS kernel summed its windows' rows whole, so

@@ -1193,6 +1193,17 @@ int finish_spmm(SpmmBuild& bd, int32_t blk_dtype, int32_t scatter_max, StilePlan
   d.tc_scale = tc_scale.empty() ? nullptr : dptr<float>(plan, o_scale);
   d.res_ptr = dptr<int32_t>(plan, o_resptr);
   d.nnz_sparse_only = res_ptr[(size_t)W * 16] - res_ptr[(size_t)W_tc * 16];
+  int64_t even_cost = 0;  // of hyb_spmm_even_rows_kernel: four rows a wave, the longest counts
+  int32_t even_longest = 0;
+  for (size_t sl = (size_t)W_tc * 16; sl < (size_t)W * 16; sl += 4) {
+    int32_t n = 0;
+    for (size_t r = sl; r < sl + 4; ++r) n = std::max(n, res_ptr[r + 1] - res_ptr[r]);
+    even_cost += 4 * n;
+    even_longest = std::max(even_longest, n);
+  }
+  d.even_rows = even_longest <= stile::kSplitNnz &&
+                (int64_t)d.nnz_sparse_only >= (int64_t)(W - W_tc) * 16 * stile::kEvenMean &&
+                even_cost * 100 <= (int64_t)d.nnz_sparse_only * stile::kEvenPercent;
   d.res_cols = dptr<int32_t>(plan, o_rescols);
   d.res_vals = dptr<float>(plan, o_resvals);
   plan->has_ids = bd.has_ids;

@@ -85,6 +85,68 @@ __global__ __launch_bounds__(256, 4) void hyb_spmm_rows_kernel(
     run(0.f);
 }
 
+// Sparse-only rows of much the same lengths, FP32 B, aligned (even_rows): one row per
+// 16-lane group and 64 columns, four columns per lane, column chunk by column chunk.
+// Bound: the gather instructions; one of 16 bytes per lane brings four entries' 256
+// bytes, where hyb_spmm_rows_kernel's brings 512 bytes of one entry.  That pays where
+// the four rows end together (their wave goes on to the longest's end).  8192 x 4000,
+// 600,000 uniform nonzeros, N = 128: 18.5 us, 23.4 by row tasks (19.1 with ids and
+// gathers not as far ahead); 262144 x 262144, 5 M, N = 256: 713 and 764.
+__global__ __launch_bounds__(256, 7) void hyb_spmm_even_rows_kernel(
+    int slot0, int nslots, const int32_t* __restrict__ res_ptr, const int32_t* __restrict__ cols,
+    const float* __restrict__ vals, const int32_t* __restrict__ win_rows, const float* __restrict__ B, int64_t ldb,
+    int N, float* __restrict__ C, int64_t ldc, int nC) {
+  const int wave = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int waves = nslots / 4;  // slots of whole windows
+  const int cch = wave / waves;
+  if (cch >= nC) return;
+  const int lane = threadIdx.x & 63;
+  const int slot = slot0 + 4 * (wave - cch * waves) + (lane >> 4);
+  const int col = cch * 64 + 4 * (lane & 15);
+  const int row = win_rows[slot], r0 = res_ptr[slot], r1 = res_ptr[slot + 1];
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (r0 < r1) {
+    // A step's ids and values are two loads each (kRowPad entries lie behind the
+    // arrays); positions past the row's end gather its last B row and are not added.
+    typedef int32_t i4 __attribute__((ext_vector_type(4), aligned(4)));
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    i4 k0, k1;
+    f4 v0, v1;
+    auto ids = [&](int q) {
+      k0 = *reinterpret_cast<const i4*>(cols + q);
+      k1 = *reinterpret_cast<const i4*>(cols + q + 4);
+      v0 = *reinterpret_cast<const f4*>(vals + q);
+      v1 = *reinterpret_cast<const f4*>(vals + q + 4);
+    };
+    auto step = [&](int q, auto whole) {
+      constexpr bool kWhole = decltype(whole)::value;
+      float4 b[8];
+      float v[8];
+      int last = k0[0];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        last = kWhole || q + i < r1 ? (i < 4 ? k0[i & 3] : k1[i & 3]) : last;
+        b[i] = load_b4(B, ldb, last, col, N, std::true_type{});
+        v[i] = i < 4 ? v0[i & 3] : v1[i & 3];
+      }
+      if constexpr (kWhole) ids(q + 8);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (kWhole || q + i < r1) {
+          s.x += v[i] * b[i].x;
+          s.y += v[i] * b[i].y;
+          s.z += v[i] * b[i].z;
+          s.w += v[i] * b[i].w;
+        }
+    };
+    ids(r0);
+    int q = r0;
+    for (; q + 8 <= r1; q += 8) step(q, std::true_type{});
+    if (q < r1) step(q, std::false_type{});
+  }
+  if (row >= 0) store_c4(C, ldc, row, col, N, true, s);
+}
+
 // Pieces of long rows, execution slots [pc0, pc1) (piece piece_exec[slot],
 // ordered by first column so that pieces of different rows gathering the same
 // B rows run together), column chunk by column chunk: summed in FP64 and added
@@ -236,6 +298,33 @@ hipError_t launch_sparse_rows(const SpmmPlanDev& p, const TB* B, int64_t ldb, in
                          dim3((unsigned)(((int64_t)n * nC + 3) / 4)), dim3(256), 0, s, p.row_tasks + a, n, p.res_ptr,
                          p.res_cols, p.res_vals, p.win_rows, B, ldb, bytes, N, C, ldc, nC);
     });
+    e = hipGetLastError();
+  }
+  return e;
+}
+
+// Rows are even when they hold kEvenMean entries on average and four times the
+// longest of each four comes to at most kEvenPercent of the entries: uniform draws
+// of 16 entries a row come to 129 %, R-MAT graphs to 300 % and more (their rows: 28
+// us by tasks, scale 13, N = 256, 95 one per lane group).  Nine entries a row, N = 512:
+// 16.6 us here, 15.9 by tasks.  A last chunk of fewer than 64 columns leaves lanes
+// idle, which shows once a chunk of B outgrows an L2 (65536 x 65536, 2 M, N = 100: 154
+// and 129 us; 8192 x 8192 22.2 and 24.8).  16-bit B, of which an entry's 128 columns
+// are one 256-byte gather: 25.1 and 17.2 (8192 x 8192, 671,088, N = 128).
+bool even_rows_fit(const SpmmPlanDev& p, int N, bool vec) {
+  return p.even_rows && vec && N > 64 && (N % 64 == 0 || (int64_t)p.K * 64 * 4 <= 4 << 20);
+}
+
+hipError_t launch_even_rows(const SpmmPlanDev& p, const float* B, int64_t ldb, int N, float* C, int64_t ldc,
+                            hipStream_t s) {
+  const int nC = (N + 63) / 64, s1 = p.W * 16;
+  // launches of whole windows (max_blocks)
+  const int64_t most = std::max<int64_t>(16, max_blocks(256) / nC * 16);
+  hipError_t e = hipSuccess;
+  for (int64_t a = (int64_t)p.W_tc * 16; a < s1 && e == hipSuccess; a += most) {
+    const int n = (int)std::min(most, s1 - a);
+    hipLaunchKernelGGL(hyb_spmm_even_rows_kernel, dim3((unsigned)(((int64_t)n / 4 * nC + 3) / 4)), dim3(256), 0, s,
+                       (int)a, n, p.res_ptr, p.res_cols, p.res_vals, p.win_rows, B, ldb, N, C, ldc, nC);
     e = hipGetLastError();
   }
   return e;

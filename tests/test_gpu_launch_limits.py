@@ -49,8 +49,16 @@ def _full(M, K):
 
 
 def test_sparse_rows(cuda):
-    # 2048 wave tasks of 64 entries, 32768 column chunks of 128
-    info = _run(cuda, _full(2048, 64), "only_ELL", False)
+    # 2048 wave tasks of 24 and 96 entries in turn, 32768 column chunks of 128
+    A = _full(2048, 96).toarray()
+    A[::2, 24:] = 0
+    info = _run(cuda, scipy.sparse.csr_matrix(A), "only_ELL", False)
+    assert info["num_chunks"] == 0 and info["num_split"] == 0
+
+
+def test_even_rows(cuda):
+    # 16384 rows of 64 entries, four to a wave, 16384 column chunks of 64 (2^20 columns)
+    info = _run(cuda, _full(16384, 64), "only_ELL", False, N=1 << 20)
     assert info["num_chunks"] == 0 and info["num_split"] == 0
 
 
