@@ -183,9 +183,15 @@ def sddmm(op, X, Y):
     return op.sddmm(X, Y)
 
 
-# Rows from which the tall kernel takes H^T G: below them the vendor's GEMM has
-# little to reduce (see _tall_kernel_fits).
+# Rows from which the tall kernel takes H^T G.  Below, both sides are little more
+# than their launches (2048 x 64: 14.5 us, the GEMM 19.7).
 _TALL_ROWS = 4096
+# Output entries up to which it does: the GEMM then has enough tiles of its own.  Kernel
+# / GEMM in us, M = 65552: 512 x 512 283 / 364, 768 x 768 811 / 1194, 1024 x 1024 1066 /
+# 938, 2048 x 512 1076 / 942; M = 32768, 1024 x 1024 534 / 464; M = 200000, 896 x 896
+# 3260 / 2745.  The GEMM's choice of tiles is uneven (1024 x 512, M = 65552: 557 / 507,
+# M = 40000: 329 / 398), so no line is right at every size.
+_TALL_OUT = 600_000
 
 
 def _own_memory(t):
@@ -207,12 +213,13 @@ def _tall_kernel_fits(H, G):
     device matrices, outside tracing and dispatch modes and outside a backward
     pass that is itself differentiated, with many more rows than output entries
     per side (a GEMM has one workgroup per output tile and a few splits of the
-    rows; measured at M = 32768, F = Fg = 256: 138 us against 56)."""
+    rows; M = 32768, F = Fg = 256: 138 us against 56; 32 times as many rows: M =
+    16384, F = 512 81 against 103, 16 times: F = 1024 267 against 236)."""
     if not (H.is_cuda and G.is_cuda and H.dtype == G.dtype == torch.float32 and _own_memory(H) and _own_memory(G)):
         return False
     M, F, Fg = H.shape[0], H.shape[1], G.shape[1]
     span = (1 << 32) - (1 << 20)
-    return (M >= _TALL_ROWS and 0 < F <= M // 32 and 0 < Fg <= M // 32 and F * Fg <= 1 << 20
+    return (M >= _TALL_ROWS and 0 < F <= M // 32 and 0 < Fg <= M // 32 and F * Fg <= _TALL_OUT
             and 4 * M * max(H.stride(0), F) < span and 4 * M * max(G.stride(0), Fg) < span
             and not torch.is_grad_enabled() and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and not is_in_torch_dispatch_mode())

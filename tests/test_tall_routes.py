@@ -107,3 +107,13 @@ def test_operands_without_memory_of_their_own_are_told_apart(monkeypatch, route)
     H, W, dY = _operands("cpu")
     torch.autograd.grad(tall_matmul(H, W), W, dY[0])
     assert seen[-1]
+
+
+@pytest.mark.gpu
+def test_wide_products_are_the_gemms(cuda):
+    """1024 x 1024 entries and 2048 x 512, which the GEMM has tiles enough for."""
+    with torch.no_grad():
+        H, G = torch.zeros(65552, 2048, device=cuda), torch.zeros(65552, 1024, device=cuda)
+        assert not autograd._tall_kernel_fits(H[:, :1024], G)
+        assert not autograd._tall_kernel_fits(H, G[:, :512])
+        assert autograd._tall_kernel_fits(H[:, :768], G[:, :768])
