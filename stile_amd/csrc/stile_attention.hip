@@ -106,6 +106,17 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), c, false);
 }
 
+// Whether any of eight BF16 values is an infinity or a NaN.
+__device__ __forceinline__ bool not_finite(const bf16x8& v) {
+  bool bad = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t w = pair_of(v, e);
+    bad |= (w & 0x7f80u) == 0x7f80u || (w & 0x7f800000u) == 0x7f800000u;
+  }
+  return bad;
+}
+
 // Sparse entries of a query handled per step.
 constexpr int kAttBatch = 4;
 typedef int32_t i32x4_u __attribute__((ext_vector_type(4), aligned(4)));
@@ -126,8 +137,7 @@ __global__ __launch_bounds__(64, 3) void attention_fused_kernel(AttArrays p, Att
                                                                 const __bf16* __restrict__ Qm,
                                                                 const __bf16* __restrict__ Km,
                                                                 const __bf16* __restrict__ Vm, int64_t ld,
-                                                                float scale, float* __restrict__ out, int64_t ldo,
-                                                                uint32_t vbytes) {
+                                                                float scale, float* __restrict__ out, int64_t ldo) {
   // the chunk's 32 K and 32 V rows; after them the sums on their way to the sparse part
   __shared__ __align__(16) unsigned char stage[64 * kAttVRow];
   static_assert(64 * kAttVRow >= 4 * 16 * kAttOStride);
@@ -300,6 +310,7 @@ __global__ __launch_bounds__(64, 3) void attention_fused_kernel(AttArrays p, Att
   // entry's probability is rounded to BF16 against the maximum of the row so
   // far, entry by entry, and then brought to the step's.
   {
+    const bf16x8 z0 = row8(Vm, row_off(0, 16 * s4)), z1 = row8(Vm, row_off(0, 16 * s4 + 64));
     float* const os = reinterpret_cast<float*>(stage);  // [16][kAttOStride]
 #pragma unroll
     for (int t = 0; t < 4; ++t)
@@ -311,7 +322,11 @@ __global__ __launch_bounds__(64, 3) void attention_fused_kernel(AttArrays p, Att
       const float4 v = ld4(os + sq * kAttOStride + 8 * s4 + (e < 8 ? e : 24 + e));
       om[e] = v.x; om[e + 1] = v.y; om[e + 2] = v.z; om[e + 3] = v.w;
     }
-    const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(Vm), 0, vbytes, 0x00020000);
+    // Entries past a row's end read V's row 0 with probability 0: where that holds an
+    // infinity or a NaN (0 times it is a NaN) their values are zeroed.  (3 masks of
+    // 2,646 rows, 64 of 640 to 5,120: 11.6 and 77.0 us, 11.4 and 76.8 without; zeroed
+    // always 11.6 and 77.2, by loads past a descriptor of V 12.2 and 77.0.)
+    const bool spoilt = __any(not_finite(z0) || not_finite(z1));
     for (int j = 0; j < n; j += kAttBatch) {
       bf16x8 ka[kAttBatch], kb[kAttBatch], va[kAttBatch], vb[kAttBatch];
       bool on[kAttBatch];
@@ -321,17 +336,8 @@ __global__ __launch_bounds__(64, 3) void attention_fused_kernel(AttArrays p, Att
         const Off off = row_off(on[u] ? sid[u] : 0, 16 * s4);
         ka[u] = row8(Km, off);
         kb[u] = row8(Km, off + 64);
-        // V of entries past a row's end is 0, whatever the rows hold (0 times an
-        // infinity or a NaN is a NaN): loads past the descriptor (64 masks of 640
-        // to 5,120 rows: 78.9 us a pass), or selects below (79.9)
-        if constexpr (kSmall) {
-          const uint32_t voff = on[u] ? off : vbytes;
-          va[u] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(vr, voff, 0, 0));
-          vb[u] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(vr, voff + 64, 0, 0));
-        } else {
-          va[u] = row8(Vm, off);
-          vb[u] = row8(Vm, off + 64);
-        }
+        va[u] = row8(Vm, off);
+        vb[u] = row8(Vm, off + 64);
       }
       load_cols(j + kAttBatch);
       __builtin_amdgcn_sched_barrier(0);  // every load of the step before its arithmetic
@@ -345,12 +351,10 @@ __global__ __launch_bounds__(64, 3) void attention_fused_kernel(AttArrays p, Att
         sval[u] = on[u] ? dot : -INFINITY;
         m_run = fmaxf(m_run, sval[u]);
       }
-      if constexpr (!kSmall) {
-        if (!__all(on[kAttBatch - 1])) {
+      if (spoilt) {
 #pragma unroll
-          for (int u = 0; u < kAttBatch; ++u)
-            if (!on[u]) va[u] = vb[u] = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
-        }
+        for (int u = 0; u < kAttBatch; ++u)
+          if (!on[u]) va[u] = vb[u] = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
       }
       auto prob = [&](float x, float mx) { return x == -INFINITY ? 0.f : __expf((x - mx) * scale); };
       if (__all(m_run == ms)) {
@@ -406,16 +410,15 @@ hipError_t launch_attention(const SpmmPlanDev& p, const AttOrder& ord, const voi
   int longest = 0;
   for (int x = 0; x < kXcds; ++x) longest = max(longest, ord.start[x + 1] - ord.start[x]);
   // 32-bit row offsets from 24-bit products: up to 2^24 rows and 4 GiB (of Q: M,
-  // of K and V: K, equal in attention plans), less a row so that offsets past V
-  // stay below 2^32
+  // of K and V: K, equal in attention plans)
   const int64_t rows = max(p.M, p.K);
-  const bool small = rows < (1 << 24) && ld < (1 << 23) && rows * ld * 2 < ((int64_t)1 << 32) - 256;
+  const bool small = rows < (1 << 24) && ld < (1 << 23) && rows * ld * 2 < ((int64_t)1 << 32);
   const auto kernel = small ? attention_fused_kernel<true> : attention_fused_kernel<false>;
   const AttArrays arrays{p.win_rows, p.tc_ptr, p.tc_cols, p.tc_mask, p.res_ptr, p.res_cols};
   auto launch = [&](const AttOrder& o, int most) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)(most * kXcds)), dim3(64), 0, s, arrays, o,
                        static_cast<const __bf16*>(Q), static_cast<const __bf16*>(K), static_cast<const __bf16*>(V),
-                       ld, scale, out, ldo, small ? (uint32_t)((p.K - 1) * ld * 2 + 128) : 0u);
+                       ld, scale, out, ldo);
     return hipGetLastError();
   };
   constexpr int kMost = (int)(max_blocks(64) / kXcds);  // windows per XCD of one launch
