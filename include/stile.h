@@ -150,11 +150,13 @@ typedef struct {
   int64_t block_nnz;      /* nonzeros carried by MFMA blocks */
   int64_t sparse_nnz;     /* nonzeros carried by the FP32 1D/ELL path */
   int64_t device_bytes;   /* bytes of plan buffers resident on the device */
-  int32_t hub_rows;       /* rows with > 4096 sparse nonzeros: each 256-term
-                             piece of such a row is summed in FP64, the
-                             pieces then added in FP32 */
+  int32_t hub_rows;       /* rows with > 4096 sparse nonzeros: their first 256
+                             terms are summed in FP64 by the row tasks
+                             (compensated FP32 where few rows run one to a
+                             wave), the rest in pieces */
   int32_t num_split;      /* SpMM: pieces of rows with > 256 sparse nonzeros,
-                             added to C by the pieces kernel */
+                             each summed in FP64 and added to C in FP32 by the
+                             pieces kernel */
 } StilePlanInfo;
 
 /* ---------------------------------------------------------------------------

@@ -7,10 +7,12 @@
 
 namespace stile {
 
-// Hub rows: a row whose sparse (non-MFMA) part has more than this many
-// nonzeros is summed in FP64 per kSplitNnz-term piece (the pieces are then
-// added plainly in FP32); the plain CSR kernels and the one-wave-per-row
-// kernel of few rows sum it with compensated (Neumaier) FP32 arithmetic.
+// Hub rows: the first kSplitNnz terms of a row whose sparse (non-MFMA) part has
+// more than this many nonzeros are summed in FP64 by the row tasks, with
+// compensated (Neumaier) FP32 arithmetic by the one-wave-per-row kernel of few
+// rows and the B-stationary launch's tail.  (The pieces of every split row are
+// summed in FP64 and added plainly in FP32.)  The plain CSR kernels sum such rows
+// whole with compensated arithmetic.
 constexpr int kHubNnz = 4096;
 
 // Rows whose sparse part is longer than this are cut: the window pass sums

@@ -230,10 +230,11 @@ hipError_t launch_csr_sddmm_f32(int M, int nnz, int Kf, const int32_t* indptr,
 // Kernels of one run, in stream order.  Plans on the B-stationary kernel
 // (BF16 blocks, K <= kLdsMaxK): that kernel computes every dense window with
 // its sparse part, and as its tail (when they are few) the sparse-only rows;
-// otherwise the sparse-row kernels run the sparse-only rows.  Other plans: the
-// streaming kernel (stile_stream.hip) stores the dense windows, with their
-// sparse parts when those are short, and the sparse-row kernels
-// (stile_sparse.hip) add the longer ones and write the sparse-only windows.
+// otherwise the sparse-row kernels run the sparse-only rows.  Other plans: a
+// streaming kernel (stile_stream.hip) stores the dense windows, with their sparse
+// parts when those are few and short and the launch does not fill the GPU, and the
+// sparse-row kernels (stile_sparse.hip) add the others and write the sparse-only
+// windows.
 // Last, the pieces of rows longer than kSplitNnz: added with atomicAdd, or, in
 // the deterministic mode, summed into a workspace and added by a reduce kernel.
 //

@@ -14,8 +14,10 @@ namespace stile {
 constexpr int kSddmmU = 4;
 // With more features than this the four waves of a workgroup share a dense block:
 // one wave waits for Kf / 64 steps of loads in sequence (R-MAT scale 15, K = 163:
-// 44.7 us, shared 34.4).  Up to 128 features (attention heads) the sum stays one
-// wave's, in the order of the features.
+// 44.7 us, shared 34.4).  The line is not where sharing stops to pay (K = 64 13.4 us
+// alone, 12.0 shared; 128 21.9 and 19.9): up to 128 features, attention heads, the
+// sum stays one wave's in the order of the features, so that scores a softmax rounds
+// to BF16 do not move.
 constexpr int kSharedKf = 128;
 
 // Sum over aligned segments of LPE <= 16 lanes, left in every lane: lanes 8, 4, 2

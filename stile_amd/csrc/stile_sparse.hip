@@ -244,8 +244,7 @@ namespace {
 // 161 us.  Sixteen entries a batch: 265 us, the scalar registers spill.  One
 // slice of columns per XCD: no change.)
 //
-// FP32 B whose 128 columns are more than twice the L2s together (8 x 4 MB): 1 as
-// well.  The launch runs column chunk by column chunk, and what one chunk's
+// FP32 B whose 128 columns are more than kWideBytes: 1 as well.  The launch runs column chunk by column chunk, and what one chunk's
 // gathers touch, half as much of B, is then found in L2 and MALL more often.  A
 // graph's whole product, FP32, N = 128, two columns per lane / one: scale 18 (128
 // columns are 128 MB) 430 / 366 us; 19: 938 / 793; 20: 2005 / 1709, N = 256 4000
@@ -253,6 +252,8 @@ namespace {
 // 183, sparse only 173 / 175, N = 200 306 / 332), smaller ones lose (16, N = 256:
 // 166 / 172).  16-bit B, whose two columns are those 256 bytes a gather, keeps
 // two at every size: scale 17 125 / 170, 20 1070 / 1297.
+// The line lies at 64 MB, where K = 131,072 (scale 17) is the last to take two: both
+// widths are within 9 % of each other there, with the sign changing by plan and N.
 constexpr int64_t kFewWaves = 2048;
 constexpr int64_t kWideBytes = 64 << 20;
 int row_width(int N, int K, int elem, int64_t waves) {
